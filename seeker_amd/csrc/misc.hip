@@ -226,8 +226,8 @@ __global__ __launch_bounds__(64) void k_prep16_swiglu(PrepArgs a) {
 int sh_prep_launch(sh_engine* e, const PrepArgs& a) {
   SH_CHECK(a.K % 32 == 0, SH_ERR_ARG, "prep K=%u not a multiple of 32", a.K);
   if (a.bh) {
-    SH_CHECK(a.N >= 1 && a.N <= SH_MAX_COLS16 && a.ldb >= a.K, SH_ERR_ARG,
-             "f16 prep N=%u (at most %u), ldb %u < K %u", a.N, SH_MAX_COLS16, a.ldb, a.K);
+    SH_CHECK(a.N >= 1 && a.N <= SH_MAX_COLS_T && a.ldb >= a.K, SH_ERR_ARG,
+             "f16 prep N=%u (at most %u), ldb %u < K %u", a.N, SH_MAX_COLS_T, a.ldb, a.K);
     SH_CHECK(a.part_cols >= a.N || a.nparts == 0, SH_ERR_ARG, "prep: partials hold %u columns, N=%u", a.part_cols,
              a.N);
     SH_CHECK(a.mode == PREP_SWIGLU ? (a.part && a.nparts > 0) : a.x != nullptr, SH_ERR_ARG, "prep inputs missing");

@@ -2327,8 +2327,10 @@ extern "C" int sh_gemm_wide16(sh_engine* e, const sh_qtensor* w, const float* x_
   SH_CHECK((w->m.type == GGML_Q4_K && w->m.K % 256 == 0) || sh_gemm16x_ok(w->m), SH_ERR_UNSUPPORTED,
            "sh_gemm_wide16: Q4_K, Q5_K, Q6_K (K a multiple of 256) or Q8_0 (of 32); type %d, K %u", w->m.type,
            w->m.K);
-  const uint32_t K = w->m.K, M = w->m.M, CW = SH_MAX_COLS16;
-  const size_t part_floats = sh_gemm16_part_floats(w->m);
+  // passes as even as the widest one allows, in whole 32-column groups
+  const uint32_t K = w->m.K, M = w->m.M, most = sh_gemm16_max_cols(w->m), npass = (N + most - 1) / most;
+  const uint32_t CW = std::min(most, ((N + npass - 1) / npass + 31) / 32 * 32);
+  const size_t part_floats = sh_gemm16_part_floats(w->m, CW);
   uint16_t* bh = nullptr;
   float* part = nullptr;
   SH_HIP(hipMallocAsync((void**)&bh, (size_t)CW * K * 2, e->stream));
@@ -2340,6 +2342,12 @@ extern "C" int sh_gemm_wide16(sh_engine* e, const sh_qtensor* w, const float* x_
     pr.mode = PREP_PLAIN; pr.x = const_cast<float*>(x_dev + (size_t)c0 * K); pr.K = K; pr.N = nc;
     pr.bh = bh; pr.ldb = K;
     if ((rc = sh_prep_launch(e, pr))) break;
+    if (sh_gemm16_splits(w->m, nc) == 1) {  // whole sums: straight into y
+      EpiArgs st;
+      st.out = y_dev + (size_t)c0 * M; st.ldo = M; st.rows = M;
+      rc = sh_gemm16_launch(e, w->m, bh, K, nc, accumulate ? EPI_ADD : EPI_STORE, st, "gemm16");
+      continue;
+    }
     EpiArgs pa;
     pa.out = part; pa.ldo = w->m.tiles * 16;
     pa.part_stride = (size_t)ncp * pa.ldo;

@@ -29,12 +29,25 @@ __device__ __forceinline__ void sh_dma16(const void* src, const void* lds) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(sh_lds_addr(lds))
                : "memory", "m0");
 }
+// 16 bytes per lane from a wave-uniform base plus the lane's byte offset.
+__device__ __forceinline__ void sh_dma16_s(const void* base, uint32_t off, const void* lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(sh_lds_addr(lds))
+               : "memory", "m0");
+}
 // 4 bytes per lane.
 __device__ __forceinline__ void sh_dma4(const void* src, const void* lds) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(sh_lds_addr(lds))
                : "memory", "m0");
 }
 // The same with the non-temporal hint, for streams read once (weights).
+__device__ __forceinline__ void sh_dma16_snt(const void* base, uint32_t off, const void* lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(base), "s"(sh_lds_addr(lds))
+               : "memory", "m0");
+}
+__device__ __forceinline__ void sh_dma4_snt(const void* base, uint32_t off, const void* lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1 nt" ::"v"(off), "s"(base), "s"(sh_lds_addr(lds))
+               : "memory", "m0");
+}
 __device__ __forceinline__ void sh_dma16_nt(const void* src, const void* lds) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(src), "s"(sh_lds_addr(lds))
                : "memory", "m0");
@@ -50,3 +63,7 @@ template <int N>
 __device__ __forceinline__ void sh_wait_vm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
+// A barrier that publishes LDS without draining the loads in flight (a
+// __syncthreads() may wait for all of them): this wave's LDS reads are done
+// (its buffers may be refilled) before it arrives.
+__device__ __forceinline__ void sh_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }

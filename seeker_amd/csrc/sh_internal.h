@@ -64,6 +64,8 @@ constexpr uint32_t SH_MAX_PREP_COLS = 512;  // operand columns one prep builds (
 constexpr int SH_FA_MIN_SPLIT_KEYS = 64;  // smallest key split of any attention launch (sizes fa_part)
 constexpr uint32_t SH_WIDE16_COLS = 32;  // the reference's wide-GEMM threshold (ops/matmul.rs:433-446)
 constexpr uint32_t SH_MAX_COLS16 = 192;  // columns per forward chunk of a wide f16 call (12 MFMA groups of 16)
+constexpr uint32_t SH_MAX_COLS_T = 2048;  // columns of one pass of the large-tile wide GEMM (k_gemm16t)
+constexpr size_t SH_PART16_BYTES = 64u << 20;  // most split partials of a wide f16 GEMM (above, fewer splits)
 constexpr int SH_FA_MAX_ROWS = 256;       // padded query rows (gqa x columns) per kv head
 // Split partial row: O[hd], m, l, 2 pad (keeps rows 16-byte aligned).
 __host__ __device__ constexpr uint32_t sh_fa_part_stride(uint32_t hd) { return hd + 4; }
@@ -373,13 +375,27 @@ int sh_gemm_launch(sh_engine* e, const QMat& w, const uint16_t* bx, const uint16
                    EpiKind epi, const EpiArgs& ea, const char* tag, uint32_t* nparts = nullptr);
 size_t sh_gemm_part_floats(const QMat& w);  // for SH_MAX_COLS columns
 // y = W x with the reference's wide-GEMM arithmetic (f16 weights and
-// activations, f32 accumulation) for N <= SH_MAX_COLS16 columns of f16 rows
-// bh[col * ldb + k] (k_prep16_*), W Q4_K, Q5_K, Q6_K or Q8_0: EPI_PART
+// activations, f32 accumulation) for N <= sh_gemm16_max_cols(w) columns of f16
+// rows bh[col * ldb + k] (k_prep16_*), W Q4_K, Q5_K, Q6_K or Q8_0: EPI_PART
 // (partials as sh_gemm_launch's; *nparts = splits) or EPI_STORE (out[col][row]).
+// Where sh_gemm16_splits(w, N) is 1 the launch covers whole sums with EPI_PART
+// as well, and EPI_STORE / EPI_ADD (out[col][row] += ...) save the partials;
+// 0: another kernel takes the call.
+uint32_t sh_gemm16_max_cols(const QMat& w);
+uint32_t sh_gemm16_splits(const QMat& w, uint32_t N);
 int sh_gemm16_launch(sh_engine* e, const QMat& w, const uint16_t* bh, uint32_t ldb, uint32_t N, EpiKind epi,
                      const EpiArgs& ea, const char* tag, uint32_t* nparts = nullptr);
-// Partial floats sh_gemm16_launch's EPI_PART needs for up to SH_MAX_COLS16 columns.
-size_t sh_gemm16_part_floats(const QMat& w);
+// Partial floats sh_gemm16_launch's EPI_PART needs for calls of up to `most`
+// columns.
+size_t sh_gemm16_part_floats(const QMat& w, uint32_t most = SH_MAX_COLS16);
+// The large-tile kernel of the same arithmetic (gemm16t.hip): 256 rows x 32 CG
+// columns per workgroup in ncb column blocks, KS splits of HS half superblocks.
+struct Gemm16tPlan {
+  uint32_t CG = 8, ncb = 1, HS = 0, KS = 1;
+};
+Gemm16tPlan sh_gemm16t_plan(const QMat& w, bool one_split, uint32_t N);
+int sh_gemm16t_launch(sh_engine* e, const QMat& w, const uint16_t* bh, uint32_t ldb, uint32_t N, const Gemm16tPlan& p,
+                      EpiKind epi, const EpiArgs& ea);
 // The same arithmetic for Q8_0, Q5_K and Q6_K weights (gemm16x.hip), which
 // sh_gemm16_launch hands these types to: whether w takes it, its partial
 // floats, the launch.

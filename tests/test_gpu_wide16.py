@@ -91,3 +91,18 @@ def test_wide16_other_formats(engine, qtype, M, K, N):
     print(f"  vs or_gemv16 {err:.2e}, vs exact {dex:.2e}", flush=True)
     assert err < 1e-5, err
     assert dex > 4 * err
+
+
+# The large-tile kernel (gemm16t.hip; 256 rows x 32 CG columns per workgroup) at
+# its edges: one superblock, ragged rows and columns, partly filled row blocks
+# and column blocks, several splits, more than one pass of 2048 columns. Bound
+# as test_wide16_small's (same operands, same f32 sums).
+@pytest.mark.parametrize("M,K,N,acc", [(37, 256, 193, True), (300, 1280, 129, False), (4100, 512, 321, False),
+                                       (2816, 512, 1025, True), (272, 768, 2081, False), (256, 4096, 257, True)])
+def test_wide16_large_tile(engine, M, K, N, acc):
+    got, ref, exact = _run(engine, M, K, N, seed=M + N, accumulate=acc)
+    scale = np.abs(ref).max()
+    err, dex = np.abs(got - ref).max() / scale, np.abs(got - exact).max() / scale
+    print(f"  vs or_gemv16 {err:.2e}, vs exact {dex:.2e}", flush=True)
+    assert err < 2e-5, err
+    assert dex > 2 * err
