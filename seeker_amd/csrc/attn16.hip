@@ -42,6 +42,7 @@
 
 #include "sh_internal.h"
 #include "sh_coherent.h"
+#include "sh_dma.h"
 #include "sh_operand.h"
 
 namespace {
@@ -376,13 +377,208 @@ __global__ __launch_bounds__(256) void k_fa16_chain(Fa16Args a, float* __restric
   if (t >= 64) return;
   const float4 v = make_float4(outf[4 * t], outf[4 * t + 1], outf[4 * t + 2], outf[4 * t + 3]);
   const uint32_t k = 256 * sb + 4 * t;
-  if (k < Dq) *(float4*)(attn + (size_t)(a.col0 + c) * Dq + k) = v;
+  if (attn && k < Dq) *(float4*)(attn + (size_t)(a.col0 + c) * Dq + k) = v;
   if (bh) {
     const h4 h = {(_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
     if (k < Dq) *(uint2*)(bh + (size_t)(a.col0 + c) * Dq + k) = __builtin_bit_cast(uint2, h);
   } else {
     sh_operand_store_sb(v, Dq, sb, a.col0 + c, bx, xs, cs);
   }
+}
+
+// The same arithmetic, bit for bit, with the blocks in order in one workgroup:
+// for calls of enough columns that the query rows alone fill the chip (prefill).
+// A workgroup of 4 waves covers 128 query rows of a kv head, wave w rows
+// 32 w .. +31 (two 16-row tiles), and walks the 64-key blocks of its rows once:
+// per block S, the running maximum, P16, the f16 P V accumulator and the chain
+// step, the f16 output in registers. Nothing per block goes to memory (the split
+// kernels write and read 256 B per row and block). K and V blocks go through two
+// LDS buffers in fragment order by direct loads, one block ahead of the compute.
+// Bound by the vector instructions: rounding the P V accumulator to f16 after
+// every 16-key chunk and the softmax are ~850 per wave and block against 96
+// MFMAs, so K / V loads and MFMAs hide behind them (two waves per SIMD).
+// Longest rows first, paired with the shortest on the second half of the grid.
+template <int HD>
+__global__ __launch_bounds__(256, 2) void k_fa16_rows(Fa16Args a, float* __restrict__ attn, uint16_t* __restrict__ bh) {
+  constexpr int NC = HD / 32, DT = HD / 16, KF = 4 * NC, NF = KF + 2 * DT;  // K and V fragments of a block
+  __shared__ h8 skv[2][NF * 64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, r = lane & 15;
+  const uint32_t R = a.gqa * a.ncol, nw = (R + 127) / 128, half = (nw + 1) / 2;
+  const uint32_t kh = blockIdx.x % a.n_kv, x = blockIdx.x / a.n_kv;
+  const uint32_t rgw = x < half ? nw - 1 - x : x - half;
+  const uint32_t rho0 = 128 * rgw + 32 * wave, Dq = a.n_head * HD;
+  auto blocks = [&](uint32_t rho) { return min(a.mask_base + rho / a.gqa, a.kvlen - 1) / 64 + 1; };
+  const uint32_t nb = blocks(min(128 * rgw + 127, R - 1));                     // the workgroup's blocks
+  const uint32_t nbw = rho0 < R ? blocks(min(rho0 + 31, R - 1)) : 0u;          // the wave's
+  const uint32_t full = rho0 < R ? (a.mask_base + rho0 / a.gqa + 1) / 64 : 0u;  // blocks without a masked key
+
+  const uint16_t* kbase = a.kc + (size_t)kh * a.max_seq * HD;
+  const uint16_t* vbase = a.vc + (size_t)kh * (a.max_seq / 32) * HD * 32;
+  auto issue = [&](uint32_t j, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NF / 4; ++i) {
+      const int f = wave + 4 * i;
+      if (f < KF) {
+        const uint32_t key = min(64 * j + 16 * (f / NC) + r, a.max_seq - 1);
+        sh_dma16_s(kbase, (key * HD + 32 * (f % NC) + 8 * g) * 2, &skv[buf][f * 64]);
+      } else {
+        const uint32_t vb = min(2 * j + (f - KF) / DT, a.max_seq / 32 - 1);
+        sh_dma16_s(vbase, ((vb * HD + 16 * ((f - KF) % DT) + r) * 32 + 8 * g) * 2, &skv[buf][f * 64]);
+      }
+    }
+  };
+  issue(0, 0);
+
+  h8 qop[2][NC];
+  uint32_t col[2];
+  bool rok[2];
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+    const uint32_t rho = rho0 + 16 * rt + r;
+    rok[rt] = rho < R;
+    const uint32_t rr = rok[rt] ? rho : 0u;
+    col[rt] = rr / a.gqa;
+    const float* qp = a.q + (size_t)col[rt] * Dq + (size_t)(kh * a.gqa + rr % a.gqa) * HD + 8 * g;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const f4 x0 = *(const f4*)(qp + 32 * c), x1 = *(const f4*)(qp + 32 * c + 4);
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        float y = (t < 4 ? x0[t & 3] : x1[t & 3]) * a.qs;
+        asm volatile("" : "+v"(y));  // the f32 product, not a fused multiply-convert
+        qop[rt][c][t] = (_Float16)y;
+      }
+    }
+  }
+  h2 o[2][DT][2];
+  float M[2], L[2];
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+    M[rt] = kNegBig;
+    L[rt] = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) o[rt][dt][0] = o[rt][dt][1] = h2{(_Float16)0.f, (_Float16)0.f};
+  }
+
+  for (uint32_t j = 0; j < nb; ++j) {
+    sh_wait_vm<0>();
+    sh_lds_barrier();  // block j is in its buffer, everyone is done with block j - 1's
+    if (j + 1 < nb) issue(j + 1, (j + 1) & 1);
+    if (j >= nbw) continue;  // wave-uniform: its rows end here
+    const h8* sk = skv[j & 1];
+    const h8* sv = sk + KF * 64;
+    f4 s[4][2];
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) {
+      h8 kop[NC];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) kop[c] = sk[(kt * NC + c) * 64 + lane];
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt) {
+        f4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kop[c], qop[rt][c], acc, 0, 0, 0);
+        s[kt][rt] = acc;
+      }
+    }
+    if (j >= full) {
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            const bool vis = fa16_visible(64 * j + 16 * kt + 4 * g + t, a.kvlen, a.mask_base, col[rt]);
+            s[kt][rt][t] = vis ? s[kt][rt][t] : -INFINITY;
+          }
+    }
+    h4 pk[4][2];
+    _Float16 e16[2];
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      float m = kNegBig;
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) m = fmaxf(m, s[kt][rt][t]);
+      m = fmaxf(m, __shfl_xor(m, 16));
+      m = fmaxf(m, __shfl_xor(m, 32));
+      m = fmaxf(M[rt], m);
+      float ps = 0.f;
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const float p = __builtin_amdgcn_exp2f(s[kt][rt][t] - m);  // 0 where masked
+          ps += p;
+          pk[kt][rt][t] = (_Float16)p;
+        }
+      ps += __shfl_xor(ps, 16);
+      ps += __shfl_xor(ps, 32);
+      const float e = __builtin_amdgcn_exp2f(M[rt] - m);
+      L[rt] = e * L[rt] + ps;
+      M[rt] = m;
+      e16[rt] = (_Float16)e;
+    }
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      const h8 v0 = sv[dt * 64 + lane], v1 = sv[(DT + dt) * 64 + lane];
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt) {
+        f4 acc = {0.f, 0.f, 0.f, 0.f};
+        h4 p16;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+          const h8 v8 = kt < 2 ? v0 : v1;
+          const h4 va = (kt & 1) ? h4{v8[4], v8[5], v8[6], v8[7]} : h4{v8[0], v8[1], v8[2], v8[3]};
+          acc = __builtin_amdgcn_mfma_f32_16x16x16f16(va, pk[kt][rt], acc, 0, 0, 0);
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {  // the f16 accumulator
+            p16[t] = (_Float16)acc[t];
+            acc[t] = (float)p16[t];
+          }
+        }
+        const h2 e2 = {e16[rt], e16[rt]};
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          h2 y = o[rt][dt][u] * e2;  // f16(f16(e) O16)
+          asm volatile("" : "+v"(y));  // two roundings, not a fused multiply-add
+          o[rt][dt][u] = y + h2{p16[2 * u], p16[2 * u + 1]};  // f16(O16 + PV16)
+        }
+      }
+    }
+  }
+
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+    if (!rok[rt]) continue;
+    const uint32_t rho = rho0 + 16 * rt + r;
+    const float il = L[rt] == 0.f ? 0.f : 1.0f / L[rt];
+    const size_t at = (size_t)(a.col0 + col[rt]) * Dq + (size_t)(kh * a.gqa + rho % a.gqa) * HD + 4 * g;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      const h2 x = o[rt][dt][0], y = o[rt][dt][1];
+      const float4 v = make_float4((float)x[0] * il, (float)x[1] * il, (float)y[0] * il, (float)y[1] * il);
+      if (attn) *(float4*)(attn + at + 16 * dt) = v;
+      const h4 h = {(_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
+      *(uint2*)(bh + at + 16 * dt) = __builtin_bit_cast(uint2, h);
+    }
+  }
+}
+
+// Which kernels take a wide call (f16 operand rows). One pass costs ~2.5 us per
+// 64-key block of the longest row whatever the number of rows (up to 400
+// workgroups), the split kernels ~17 us more to start and, per block, what
+// writing and reading the rows' PV16 takes (2.65e-4 us a query row of a kv
+// head), both at head_dim 128 and in proportion to it. Measured on the 8B shape
+// (attention + chain, us a layer): 192 columns over 192 / 1192 / 4192 keys 17 /
+// 56 / 167 against 29 / 54 / 132, 320 over 320 / 2320 22 / 98 against 47 / 129,
+// 2048 over 2048 93 against 544.
+bool use_rows(uint32_t n_kv, uint32_t hd, uint32_t rows, uint32_t kv) {
+  const double nb = (kv + 63) / 64, per = 2.5 - 2.65e-4 * rows * n_kv;
+  return nb * hd / 128.0 * per <= 17.0;
 }
 
 }  // namespace
@@ -397,11 +593,15 @@ size_t sh_fa16_sync_words(uint32_t n_kv, uint32_t gqa, uint32_t ncol, uint32_t k
   return (size_t)n_kv * n_rg * ((nbmax + kW - 1) / kW);
 }
 
+bool sh_fa16_rows(const sh_model* m, const FaArgs& fa, bool f16_rows) {
+  return f16_rows && !fa.dbase && use_rows(m->n_kv, m->hd, m->n_head / m->n_kv * fa.N, fa.kvlen);
+}
+
 int sh_fa16_launch(sh_engine* e, const sh_model* m, const sh_kv* kv, const FaArgs& fa, const float* q,
                    float* attn_out, uint16_t* bx, uint16_t* xs, float* cs, uint16_t* bh) {
   const Workspace& w = m->ws;
   const uint32_t gqa = m->n_head / m->n_kv;
-  SH_CHECK(fa.N >= 1 && fa.col0 + fa.N <= w.max_cols, SH_ERR_ARG, "cm1 attention: columns [%u, %u)", fa.col0,
+  SH_CHECK(fa.N >= 1 && fa.col0 + fa.N <= SH_MAX_COLS_T, SH_ERR_ARG, "cm1 attention: columns [%u, %u)", fa.col0,
            fa.col0 + fa.N);
   SH_CHECK(fa.kvlen > 0 || fa.dbase, SH_ERR_ARG, "attention over zero keys");
   SH_CHECK(!fa.dbase || fa.kv_cap >= fa.kvlen, SH_ERR_ARG, "attention: graph key capacity below the offset");
@@ -421,6 +621,16 @@ int sh_fa16_launch(sh_engine* e, const sh_model* m, const sh_kv* kv, const FaArg
   // q * (scale * log2 e) with scale = 1 / sqrt(head_dim), each in f32 (models/llama.rs:237)
   const float scale = 1.0f / sqrtf((float)m->hd);
   a.qs = scale * 1.44269504088896340736f;
+  if (sh_fa16_rows(m, fa, bh != nullptr)) {
+    hipEvent_t ev = nullptr;
+    sh_prof_begin(e, &ev);
+    const dim3 grid((gqa * fa.N + 127) / 128 * m->n_kv);
+    if (m->hd == 128) hipLaunchKernelGGL(k_fa16_rows<128>, grid, dim3(256), 0, e->stream, a, attn_out, bh);
+    else hipLaunchKernelGGL(k_fa16_rows<64>, grid, dim3(256), 0, e->stream, a, attn_out, bh);
+    SH_HIP(hipGetLastError());
+    sh_prof_end(e, "attention", 2.0 * m->n_kv * (double)kv_grid * m->hd * 2.0, ev);
+    return SH_OK;
+  }
   SH_CHECK(sh_fa16_pv_halves(m->n_kv, m->hd, gqa, fa.N, kv_grid) <= w.fa16_pv_halves &&
                sh_fa16_sync_words(m->n_kv, gqa, fa.N, kv_grid) <= w.fa16_sync_words,
            SH_ERR_CAPACITY, "cm1 attention buffers too small");

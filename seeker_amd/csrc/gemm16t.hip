@@ -31,6 +31,7 @@
 
 #include "sh_internal.h"
 #include "sh_dma.h"
+#include "sh_qkv.h"
 
 namespace {
 
@@ -285,6 +286,28 @@ __global__ __launch_bounds__(64 * kWaves, 1) void k_gemm16t(const uint8_t* __res
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last MFMAs' results
   __builtin_amdgcn_sched_barrier(0);
 
+  if (EPI == EPI_QKV && ea.row_base + tile0 * 16 >= ea.Dq + ea.Dkv) {
+    // V rows go out with the lanes along the columns: consecutive keys of a row
+    // are neighbours in the cache's transposed blocks
+    if (tile0 >= tiles) return;
+#pragma unroll
+    for (int c = 0; c < CG; ++c) {
+      const uint32_t col = col0 + 32 * c + (lane & 31);
+      if (col >= N) continue;
+      const QkvColDev t = ea.tab[col];
+#pragma unroll
+      for (int p = 0; p < TP; ++p)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          if (tile0 + 2 * p + q / 2 >= tiles) continue;
+          const f16v& a4 = acc[p][c];
+          const float v[4] = {a4[4 * q], a4[4 * q + 1], a4[4 * q + 2], a4[4 * q + 3]};
+          qkv_store4(ea, ea.row_base + (tile0 + 2 * p) * 16 + 8 * q + 4 * kh, v, t.pos, t.slot, t.mseq, t.kc, t.vc,
+                     nullptr);
+        }
+    }
+    return;
+  }
   // Epilogue, one column group at a time through the wave's own slice of LDS:
   // lane holds column lane % 32, rows 8 q + 4 kh + 0..3 of each pair's 32; read
   // back as 16 lanes x 4 rows of a column, so a store covers the wave's whole 64
@@ -305,11 +328,32 @@ __global__ __launch_bounds__(64 * kWaves, 1) void k_gemm16t(const uint8_t* __res
             make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
       }
     __builtin_amdgcn_wave_barrier();
+    if (EPI == EPI_SWIGLU) {  // 8 lanes cover the 32 h rows of a column's 2 gate / up pairs
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t lc = 8 * i + (lane >> 3), col = col0 + 32 * c + lc, p = (lane >> 2) & 1, rr = 4 * (lane & 3);
+        const float4 gt = *(const float4*)(st + lc * kLd + 32 * p + rr);
+        const float4 up = *(const float4*)(st + lc * kLd + 32 * p + 16 + rr);
+        if (col >= N || tile0 + 2 * p + 1 >= tiles) continue;
+        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+        const h4 h = {(_Float16)((gt.x / (1.0f + expf(-gt.x))) * up.x), (_Float16)((gt.y / (1.0f + expf(-gt.y))) * up.y),
+                      (_Float16)((gt.z / (1.0f + expf(-gt.z))) * up.z), (_Float16)((gt.w / (1.0f + expf(-gt.w))) * up.w)};
+        *(uint2*)(ea.h16 + (size_t)col * ea.ldh + (tile0 / 2 + p) * 16 + rr) = __builtin_bit_cast(uint2, h);
+      }
+      __builtin_amdgcn_wave_barrier();
+      continue;
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const uint32_t lc = 4 * i + (lane >> 4), col = col0 + 32 * c + lc;
       const float4 v = *(const float4*)(st + lc * kLd + er);
       if (col >= N || row0 >= tiles * 16) continue;
+      if (EPI == EPI_QKV) {
+        const QkvColDev t = ea.tab[col];
+        const float o[4] = {v.x, v.y, v.z, v.w};
+        qkv_store4(ea, ea.row_base + row0, o, t.pos, t.slot, t.mseq, t.kc, t.vc, ea.out + (size_t)col * ea.Dq);
+        continue;
+      }
       float* out = ea.out + (size_t)col * ea.ldo + row0;
       if (EPI == EPI_PART) {
         *(float4*)(out + ks * ea.part_stride) = v;
@@ -357,8 +401,9 @@ void dispatch(sh_engine* e, const QMat& w, const uint16_t* bh, uint32_t ldb, uin
 
 // The split plan minimises an estimate of the call's time (us, fitted to the 8B
 // shapes at 65 - 2048 columns): rounds of one workgroup per CU, each kHalf(CG)
-// per 128 k plus the fill of the pipeline and the epilogue, plus the split
-// partials' write and their read by the finishing kernel at ~4 TB/s.
+// per 128 k plus the fill of the pipeline and the epilogue, plus, with several
+// splits, the partials' write and their read at ~4 TB/s by the finishing launch
+// that a single split does without.
 Gemm16tPlan sh_gemm16t_plan(const QMat& w, bool one_split, uint32_t N) {
   const uint32_t G = (N + 31) / 32, nsb = w.K / 256, nrb = (w.tiles + 15) / 16, slots = 256;
   const size_t col_bytes = (size_t)((N + 7) / 8 * 8) * w.tiles * 16 * 4;
@@ -373,7 +418,7 @@ Gemm16tPlan sh_gemm16t_plan(const QMat& w, bool one_split, uint32_t N) {
     for (uint32_t ks = 1; ks <= cap && ks <= nsb; ++ks) {
       const uint32_t S = (nsb + ks - 1) / ks, k2 = (nsb + S - 1) / S, wgs = nrb * ncb * k2;
       if (k2 != ks) continue;
-      const double part_us = (double)(k2 - 1) * col_bytes * 2 / 4e6;
+      const double part_us = k2 > 1 ? (double)k2 * col_bytes * 2 / 4e6 + 2.0 : 0.0;
       const double cost = (double)((wgs + slots - 1) / slots) * (2 * S * (0.85 + 0.27 * even) + 8.0) + part_us;
       if (cost < best - 1e-9) {
         best = cost;
@@ -389,8 +434,16 @@ int sh_gemm16t_launch(sh_engine* e, const QMat& w, const uint16_t* bh, uint32_t 
   SH_CHECK(w.type == GGML_Q4_K && w.K % 256 == 0 && ldb >= w.K && ldb % 8 == 0 && N >= 1 && N <= 32 * p.CG * p.ncb &&
                (uint64_t)N * ldb * 2 < (1ull << 32),
            SH_ERR_ARG, "f16 gemm: type %d, K %u, ldb %u, N %u", w.type, w.K, ldb, N);
+  SH_CHECK(epi == EPI_PART || p.KS == 1, SH_ERR_ARG, "f16 gemm: epilogue %d needs whole sums", (int)epi);
+  SH_CHECK(epi != EPI_QKV || (ea.tab && ea.out && ea.hd % 4 == 0 && ea.row_base % 4 == 0 && ea.Dq % 64 == 0 &&
+                              ea.Dkv % 64 == 0 && ea.row_base + w.M <= ea.Dq + 2 * ea.Dkv),
+           SH_ERR_ARG, "f16 gemm: QKV epilogue shape");
+  SH_CHECK(epi != EPI_SWIGLU || (ea.h16 && w.tiles % 2 == 0 && ea.ldh % 4 == 0 && ea.ldh >= w.tiles * 8), SH_ERR_ARG,
+           "f16 gemm: SwiGLU epilogue shape");
   if (epi == EPI_PART) dispatch<Q4K, EPI_PART>(e, w, bh, ldb, N, p, ea);
   else if (epi == EPI_ADD) dispatch<Q4K, EPI_ADD>(e, w, bh, ldb, N, p, ea);
+  else if (epi == EPI_QKV) dispatch<Q4K, EPI_QKV>(e, w, bh, ldb, N, p, ea);
+  else if (epi == EPI_SWIGLU) dispatch<Q4K, EPI_SWIGLU>(e, w, bh, ldb, N, p, ea);
   else dispatch<Q4K, EPI_STORE>(e, w, bh, ldb, N, p, ea);
   SH_HIP(hipGetLastError());
   return SH_OK;

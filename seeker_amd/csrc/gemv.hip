@@ -30,6 +30,7 @@
 #include "sh_coherent.h"
 #include "sh_dma.h"
 #include "sh_operand.h"
+#include "sh_qkv.h"
 
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
@@ -71,12 +72,6 @@ __device__ __forceinline__ h8 q8_operand(uint32_t w0, uint32_t w1) {
   r.z = as_u32(as_h2(((b & 0xFFu) | ((b & 0xFF00u) << 8)) | 0x64006400u) + off);
   r.w = as_u32(__builtin_elementwise_fma(as_h2((((b >> 16) & 0xFFu) | ((b >> 8) & 0xFF0000u)) | 0x64006400u), k16, off16));
   return as_h8(r);
-}
-
-// Slot of key kappa (0..31) inside a 32-key V block: the PV MFMA's B operand
-// (probabilities) arrives with lane group g holding keys {4g..4g+3, 16+4g..16+4g+3}.
-__device__ __forceinline__ uint32_t v_slot(uint32_t kappa) {
-  return 8u * ((kappa & 15u) >> 2) + 4u * (kappa >> 4) + (kappa & 3u);
 }
 
 // ------------------------------------------------------------------ repack
@@ -255,41 +250,6 @@ __global__ void k_repack_q8(const uint8_t* __restrict__ src, uint8_t* __restrict
 
 
 // ------------------------------------------------------------------ epilogue
-
-__device__ __forceinline__ uint16_t f2h_bits(float x) { return __builtin_bit_cast(uint16_t, (_Float16)x); }
-
-// Rows r0..r0+3 of one column's fused QKV output: q rows are roped into
-// qcol, k rows roped and v rows stored as f16 in the column's cache slot
-// (V slot-permuted within its 32-key block).
-__device__ __forceinline__ void qkv_store4(const EpiArgs& ea, uint32_t r0, const float v[4], int32_t pos,
-                                           uint32_t slot, uint32_t ms, uint16_t* kc, uint16_t* vc, float* qcol) {
-  if (r0 < ea.Dq) {
-    const uint32_t i0 = r0 % ea.hd;
-    const float2 cs0 = ea.rope[(size_t)pos * (ea.hd / 2) + i0 / 2];
-    const float2 cs1 = ea.rope[(size_t)pos * (ea.hd / 2) + i0 / 2 + 1];
-    float* q = qcol + r0;
-    q[0] = v[0] * cs0.x - v[1] * cs0.y;
-    q[1] = v[0] * cs0.y + v[1] * cs0.x;
-    q[2] = v[2] * cs1.x - v[3] * cs1.y;
-    q[3] = v[2] * cs1.y + v[3] * cs1.x;
-  } else if (r0 < ea.Dq + ea.Dkv) {
-    const uint32_t rr = r0 - ea.Dq, kh = rr / ea.hd, i0 = rr % ea.hd;
-    const float2 cs0 = ea.rope[(size_t)pos * (ea.hd / 2) + i0 / 2];
-    const float2 cs1 = ea.rope[(size_t)pos * (ea.hd / 2) + i0 / 2 + 1];
-    float o[4];
-    o[0] = v[0] * cs0.x - v[1] * cs0.y;
-    o[1] = v[0] * cs0.y + v[1] * cs0.x;
-    o[2] = v[2] * cs1.x - v[3] * cs1.y;
-    o[3] = v[2] * cs1.y + v[3] * cs1.x;
-    uint16_t* k = kc + (((size_t)ea.layer * ea.n_kv + kh) * ms + slot) * ea.hd + i0;
-    for (int j = 0; j < 4; ++j) k[j] = f2h_bits(o[j]);
-  } else {
-    const uint32_t rr = r0 - ea.Dq - ea.Dkv, kh = rr / ea.hd, i0 = rr % ea.hd;
-    uint16_t* vb = vc + (((size_t)ea.layer * ea.n_kv + kh) * (ms / 32) + slot / 32) * ea.hd * 32;
-    const uint32_t sl = v_slot(slot & 31);
-    for (int j = 0; j < 4; ++j) vb[(size_t)(i0 + j) * 32 + sl] = f2h_bits(v[j]);
-  }
-}
 
 // Final (row, col) value for rows r0..r0+3 (one lane), col < N; ks = split.
 template <int EPI>
@@ -1948,10 +1908,16 @@ __global__ __launch_bounds__(128) void k_qkv_finish_head(const float* __restrict
       if (k0 + j < nparts) v += t[j];
   }
   const uint32_t b0 = ea.dbase ? *ea.dbase : 0u;  // graph replay: offsets from the device base
-  const int32_t pos = qc.pos[col] + (int32_t)b0;
-  const uint32_t slot = qc.slot[col] + b0, ms = qc.mseq[col];
+  QkvColDev t;
+  if (qc.tab) {
+    t = qc.tab[col];
+  } else {
+    t.pos = qc.pos[col]; t.slot = qc.slot[col]; t.mseq = qc.mseq[col]; t.kc = qc.kc[col]; t.vc = qc.vc[col];
+  }
+  const int32_t pos = t.pos + (int32_t)b0;
+  const uint32_t slot = t.slot + b0, ms = t.mseq;
   if (kind == 2) {
-    uint16_t* vb = qc.vc[col] + (((size_t)ea.layer * nkv + hh) * (ms / 32) + slot / 32) * hd * 32;
+    uint16_t* vb = t.vc + (((size_t)ea.layer * nkv + hh) * (ms / 32) + slot / 32) * hd * 32;
     vb[(size_t)i * 32 + v_slot(slot & 31)] = f2h_bits(v);
     return;  // uniform per workgroup
   }
@@ -1978,7 +1944,7 @@ __global__ __launch_bounds__(128) void k_qkv_finish_head(const float* __restrict
   if (kind == 0) {
     ea.out[(size_t)col * ea.Dq + row] = o;
   } else {
-    qc.kc[col][(((size_t)ea.layer * nkv + hh) * ms + slot) * hd + i] = f2h_bits(o);
+    t.kc[(((size_t)ea.layer * nkv + hh) * ms + slot) * hd + i] = f2h_bits(o);
   }
 }
 
@@ -2916,7 +2882,7 @@ int sh_gemm16_launch(sh_engine* e, const QMat& w, const uint16_t* bh, uint32_t l
            "f16 gemm needs Q4_K (type %d) and an operand of at least K = %u halves per column (ldb %u)", w.type, w.K,
            ldb);
   const bool t = use16t(w, N), one = epi != EPI_PART;
-  SH_CHECK(epi == EPI_PART || epi == EPI_STORE || (t && epi == EPI_ADD), SH_ERR_ARG, "f16 gemm epilogue %d", (int)epi);
+  SH_CHECK(epi == EPI_PART || epi == EPI_STORE || t, SH_ERR_ARG, "f16 gemm epilogue %d", (int)epi);
   const bool h = !t && N > SH_MAX_COLS && use16h(w, one, N);
   Gemm16tPlan pt;
   MgPlan p;
@@ -2946,7 +2912,7 @@ int sh_gemm16_launch(sh_engine* e, const QMat& w, const uint16_t* bh, uint32_t l
 
 int sh_qkv_finish_launch(sh_engine* e, const float* part, uint32_t nparts, size_t part_stride, uint32_t ldp,
                          uint32_t N, const EpiArgs& ea, const QkvCols& qc) {
-  SH_CHECK(N >= 1 && N <= (qc.tab ? (uint32_t)SH_MAX_COLS16 : (uint32_t)SH_MAX_COLS) && ea.hd % 4 == 0, SH_ERR_ARG,
+  SH_CHECK(N >= 1 && (qc.tab || N <= (uint32_t)SH_MAX_COLS) && ea.hd % 4 == 0, SH_ERR_ARG,
            "qkv finish shape");
   SH_CHECK(!(qc.tab && ea.dbase), SH_ERR_ARG, "qkv finish: a device column table has no graph base");
   SH_CHECK(qc.row0 % 4 == 0 && qc.row0 < ea.Dq + 2 * ea.Dkv && (qc.row0 < ea.Dq + ea.Dkv || qc.vpart), SH_ERR_ARG,
@@ -2964,7 +2930,7 @@ int sh_qkv_finish_launch(sh_engine* e, const float* part, uint32_t nparts, size_
 int sh_qkv_finish_head_launch(sh_engine* e, const float* part, uint32_t nparts, size_t part_stride, uint32_t ldp,
                               uint32_t N, const EpiArgs& ea, const QkvCols& qc, const float* q_norm,
                               const float* k_norm, float eps, bool neox) {
-  SH_CHECK(!qc.tab && N >= 1 && N <= SH_MAX_COLS && (ea.hd == 64 || ea.hd == 128) && ea.Dq % ea.hd == 0, SH_ERR_ARG,
+  SH_CHECK(N >= 1 && (qc.tab ? !ea.dbase : N <= SH_MAX_COLS) && (ea.hd == 64 || ea.hd == 128) && ea.Dq % ea.hd == 0, SH_ERR_ARG,
            "qkv head finish shape");
   const uint32_t heads = ea.Dq / ea.hd + 2 * ea.n_kv;
   hipEvent_t ev = nullptr;

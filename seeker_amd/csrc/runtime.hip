@@ -162,7 +162,7 @@ extern "C" int sh_engine_profile_reset(sh_engine* e) {
 }
 
 int sh_engine_scratch(sh_engine* e, int slot, size_t bytes, void** out) {
-  SH_CHECK(slot >= 0 && slot < 4, SH_ERR_ARG, "scratch slot %d", slot);
+  SH_CHECK(slot >= 0 && slot < SCR_SLOTS, SH_ERR_ARG, "scratch slot %d", slot);
   if (bytes > e->scr_bytes[slot]) {
     g_graph_gen.fetch_add(1);  // captured graphs may point into the old block
     SH_HIP(hipStreamSynchronize(e->stream));
@@ -235,7 +235,7 @@ static void free_model(sh_model* m) {
   Workspace& w = m->ws;
   (void)hipFree(w.resid); (void)hipFree(w.resid2); (void)hipFree(w.bx); (void)hipFree(w.xs); (void)hipFree(w.q);
   (void)hipFree(w.attn); (void)hipFree(w.gpart); (void)hipFree(w.h); (void)hipFree(w.logits); (void)hipFree(w.fa_part); (void)hipFree(w.fab_part);
-  (void)hipFree(w.tokens); (void)hipFree(w.amax); (void)hipFree(w.cs); (void)hipFree(w.ssq); (void)hipFree(w.bh); (void)hipFree(w.qtab);
+  (void)hipFree(w.tokens); (void)hipFree(w.amax); (void)hipFree(w.cs); (void)hipFree(w.ssq); (void)hipFree(w.bh); (void)hipFree(w.bh2); (void)hipFree(w.qtab);
   (void)hipFree(w.bx2); (void)hipFree(w.xs2); (void)hipFree(w.cs2); (void)hipFree(w.ssq2); (void)hipFree(w.sb_cnt);
   (void)hipFree(w.moe_logits); (void)hipFree(w.moe_ids); (void)hipFree(w.moe_wts); (void)hipFree(w.moe_info); (void)hipFree(w.moe_col);
   (void)hipFree(w.moe_slot); (void)hipFree(w.moe_hgu); (void)hipFree(w.moe_bx); (void)hipFree(w.moe_xs);
@@ -265,6 +265,13 @@ static int ensure_rope(sh_model* m, uint32_t npos) {
   SH_HIP(hipMemcpy(m->rope, tab.data(), tab.size() * sizeof(float2), hipMemcpyHostToDevice));
   m->rope_max = cap;
   return SH_OK;
+}
+
+// Split-partial floats of a layer's wide f16 GEMMs over calls of up to `cols`
+// columns (the V matrix's partials follow the QKV ones).
+static size_t layer_part16_floats(const Layer& L, uint32_t cols) {
+  auto f = [&](const QMat& q) { return q.d ? sh_gemm16_part_floats(q, cols) : (size_t)0; };
+  return std::max({f(L.wqkv) + f(L.wv), f(L.wo), f(L.wgu), f(L.wdown)});
 }
 
 static int load_model(sh_engine* e, const uint8_t* img, uint64_t size, sh_model** out) {
@@ -377,6 +384,10 @@ static int load_model(sh_engine* e, const uint8_t* img, uint64_t size, sh_model*
       w16 = w16 && g16(L.wqkv) && (!L.wv.d || g16(L.wv)) && g16(L.wo) &&
             (m->n_expert ? true : g16(L.wgu) && g16(L.wdown));
     m->wide16_ok = w16;
+    bool big = w16 && !m->n_expert;
+    for (const Layer& L : m->layers)
+      for (const QMat* q : {&L.wqkv, &L.wv, &L.wo, &L.wgu, &L.wdown}) big = big && (!q->d || q->type == GGML_Q4_K);
+    m->big16_ok = big;
     const char* env16 = getenv("SH_WIDE_F16");
     m->wide16 = w16 && !(env16 && atoi(env16) == 0);
     const char* envcm = getenv("SH_FA_CM");
@@ -400,15 +411,15 @@ static int load_model(sh_engine* e, const uint8_t* img, uint64_t size, sh_model*
                              sh_gemm_part_floats(L.wo), sh_gemm_part_floats(L.wgu), sh_gemm_part_floats(L.wdown)});
   if (m->wide16_ok)
     for (const Layer& L : m->layers)
-      gpart_floats = std::max({gpart_floats, sh_gemm16_part_floats(L.wqkv), sh_gemm16_part_floats(L.wo),
-                               sh_gemm16_part_floats(L.wgu), sh_gemm16_part_floats(L.wdown)});
+      gpart_floats = std::max(gpart_floats, layer_part16_floats(L, SH_MAX_COLS16));
   const size_t C = w.max_cols;
   if (dalloc(&w.resid, C * m->d) || dalloc(&w.resid2, C * m->d) || dalloc(&w.bx, bx_elems) ||
       dalloc(&w.xs, xs_elems) ||
       dalloc(&w.q, C * wide) || dalloc(&w.attn, C * wide) || dalloc(&w.gpart, gpart_floats) ||
       dalloc(&w.h, C * std::max(m->ff, 1u)) || dalloc(&w.logits, C * m->V) || dalloc(&w.fa_part, part_floats) ||
       dalloc(&w.tokens, C + 64) || dalloc(&w.amax, SH_AMAX_WORDS) || dalloc(&w.cs, ngrp * sh_grp_cs(kmax)) ||
-      dalloc(&w.ssq, ngrp * sh_grp_cs(kmax)) || dalloc(&w.bh, C * kmax) || dalloc(&w.qtab, C) || dalloc(&w.bx2, sh_grp_bx(m->d)) || dalloc(&w.xs2, sh_grp_xs(m->d)) ||
+      dalloc(&w.ssq, ngrp * sh_grp_cs(kmax)) || dalloc(&w.bh, C * kmax) ||
+      dalloc(&w.bh2, C * std::max(m->ff, 1u)) || dalloc(&w.qtab, C) || dalloc(&w.bx2, sh_grp_bx(m->d)) || dalloc(&w.xs2, sh_grp_xs(m->d)) ||
       dalloc(&w.cs2, sh_grp_cs(m->d)) || dalloc(&w.ssq2, sh_grp_cs(m->d)) || dalloc(&w.sb_cnt, SH_SB_CNT * SH_SB_CNT_STRIDE))
     FAIL(SH_ERR_HIP, "workspace allocation: %s", sh_last_error());
   w.fa_part_floats = part_floats;
@@ -1214,6 +1225,163 @@ static int forward_chunk_mg(sh_model* m, const uint32_t* dev_tokens, uint32_t nc
   return SH_OK;
 }
 
+// Where a chunk left its residual rows and the column its logits start at.
+struct ChunkOut {
+  const float* resid = nullptr;
+  uint32_t logit0 = 0;
+};
+
+// Wide f16 forward of a dense model's chunk of up to SH_MAX_COLS_T columns:
+// every matrix through sh_gemm16_launch on f16 operand rows. Where a GEMM's
+// plan has a single split its epilogue finishes the rows (RoPE and the K / V
+// writes, the residual add, SwiGLU into the down operand), so a layer of a long
+// prefill is 7 launches and no f32 partials; else split partials, finished by
+// the kernels forward_chunk_mg uses. Logits of columns lm0 .. nc - 1 only (the
+// last one of a prefill: the lm_head over all 128256 rows costs 178 us for 128
+// columns, 25 us for one). Chunks of more than w.max_cols columns use the
+// engine's scratch, sized to a power of two of columns.
+static int forward_chunk_w16(sh_model* m, const uint32_t* dev_tokens, uint32_t nc, const ColKv* cols,
+                             const std::vector<FaSeg>& segs, uint32_t lm0, bool want_resid, ChunkOut* out) {
+  sh_engine* e = m->e;
+  Workspace& w = m->ws;
+  int rc;
+  const uint32_t ncp = (nc + 7) / 8 * 8, wide = std::max(m->d, m->q_dim);
+  float *resid = w.resid, *q = w.q, *gpart = w.gpart;
+  uint16_t *bh = w.bh, *bh2 = w.bh2;
+  QkvColDev* qtab = w.qtab;
+  size_t gpart_floats = w.gpart_floats;
+  if (nc > w.max_cols) {
+    uint32_t C = 256;
+    while (C < nc) C *= 2;
+    gpart_floats = 0;
+    for (const Layer& L : m->layers) gpart_floats = std::max(gpart_floats, layer_part16_floats(L, C));
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+      const size_t o = off;
+      off += (bytes + 255) / 256 * 256;
+      return o;
+    };
+    const size_t o_resid = take((size_t)C * m->d * 4), o_q = take((size_t)C * wide * 4), o_bh = take((size_t)C * wide * 2),
+                 o_bh2 = take((size_t)C * m->ff * 2), o_tab = take((size_t)C * sizeof(QkvColDev)),
+                 o_part = take(gpart_floats * 4);
+    void* base = nullptr;
+    if ((rc = sh_engine_scratch(e, SCR_WIDE, off, &base))) return rc;
+    uint8_t* b = (uint8_t*)base;
+    resid = (float*)(b + o_resid); q = (float*)(b + o_q); bh = (uint16_t*)(b + o_bh); bh2 = (uint16_t*)(b + o_bh2);
+    qtab = (QkvColDev*)(b + o_tab); gpart = (float*)(b + o_part);
+  }
+  out->resid = resid;
+  out->logit0 = lm0;
+  if ((rc = sh_embed_launch(e, m, dev_tokens, nc, resid))) return rc;
+  std::vector<QkvColDev> tab(nc);
+  for (uint32_t j = 0; j < nc; ++j) {
+    const ColKv& c = cols[j];
+    tab[j].pos = c.pos; tab[j].slot = c.slot; tab[j].mseq = c.kv->max_seq; tab[j].pad = 0;
+    tab[j].kc = c.kv->k; tab[j].vc = c.kv->v;
+  }
+  SH_HIP(hipMemcpyAsync(qtab, tab.data(), (size_t)nc * sizeof(QkvColDev), hipMemcpyHostToDevice, e->stream));
+  EpiArgs qkv;
+  qkv.out = q; qkv.Dq = m->q_dim; qkv.Dkv = m->hd * m->n_kv; qkv.hd = m->hd; qkv.n_kv = m->n_kv; qkv.rope = m->rope;
+  qkv.tab = qtab;
+  auto part_args = [&](const QMat& mat) {
+    EpiArgs pa;
+    pa.out = gpart; pa.ldo = mat.tiles * 16;
+    pa.part_stride = (size_t)ncp * pa.ldo;
+    pa.part_cap = (uint32_t)(gpart_floats / pa.part_stride);
+    return pa;
+  };
+  uint32_t pending = 0, pending_ld = 0;  // split partials not yet added to the residual
+  // the residual (plus pending partials), normalized, as f16 rows in bh
+  auto norm_rows = [&](const float* norm_w, uint32_t c0) {
+    PrepArgs pr;
+    pr.mode = PREP_RESID; pr.x = resid + (size_t)c0 * m->d; pr.K = m->d; pr.N = nc - c0; pr.norm_w = norm_w;
+    pr.eps = m->eps; pr.part = gpart + (size_t)c0 * pending_ld; pr.part_cols = ncp; pr.part_ld = pending_ld;
+    pr.nparts = pending; pr.bh = bh; pr.ldb = m->d;
+    pending = 0;
+    return sh_prep_launch(e, pr);
+  };
+  // resid += mat x rows, or its partials pending
+  auto add_resid = [&](const QMat& mat, const uint16_t* rows, const char* tag) {
+    if (sh_gemm16_splits(mat, nc) == 1) {
+      EpiArgs ad;
+      ad.out = resid; ad.ldo = m->d; ad.rows = m->d;
+      return sh_gemm16_launch(e, mat, rows, mat.K, nc, EPI_ADD, ad, tag);
+    }
+    const EpiArgs pa = part_args(mat);
+    pending_ld = pa.ldo;
+    return sh_gemm16_launch(e, mat, rows, mat.K, nc, EPI_PART, pa, tag, &pending);
+  };
+  FabGuard fab{e, FabLaunch{}};
+  if (!m->call_cm1 && (rc = plan_fab(m, segs, nc, &fab))) return rc;
+  const bool rope4 = !m->neox && qkv.Dq % 64 == 0 && qkv.Dkv % 64 == 0;
+  for (uint32_t l = 0; l < m->n_layer; ++l) {
+    const Layer& L = m->layers[l];
+    qkv.layer = l;
+    if ((rc = norm_rows(L.attn_norm, 0))) return rc;
+    QkvCols qc;
+    qc.tab = qtab;
+    EpiArgs pq = part_args(L.wqkv);
+    uint32_t nq = 0;
+    const bool direct = rope4 && sh_gemm16_splits(L.wqkv, nc) == 1;
+    const bool direct_v = direct && L.wv.d && sh_gemm16_splits(L.wv, nc) == 1;
+    if ((rc = direct ? sh_gemm16_launch(e, L.wqkv, bh, m->d, nc, EPI_QKV, qkv, "gemv_qkv")
+                     : sh_gemm16_launch(e, L.wqkv, bh, m->d, nc, EPI_PART, pq, "gemv_qkv", &nq)))
+      return rc;
+    if (L.wv.d && direct_v) {
+      EpiArgs v = qkv;
+      v.row_base = qkv.Dq + qkv.Dkv;
+      if ((rc = sh_gemm16_launch(e, L.wv, bh, m->d, nc, EPI_QKV, v, "gemv_v"))) return rc;
+    } else if (L.wv.d) {  // v in a weight type of its own: its partials follow q / k's
+      EpiArgs pv = part_args(L.wv);
+      pv.out = gpart + nq * pq.part_stride;
+      pv.part_cap = (uint32_t)((gpart_floats - nq * pq.part_stride) / pv.part_stride);
+      if ((rc = sh_gemm16_launch(e, L.wv, bh, m->d, nc, EPI_PART, pv, "gemv_v", &qc.vnparts))) return rc;
+      qc.vpart = pv.out; qc.vldp = pv.ldo; qc.vstride = pv.part_stride;
+    }
+    if (!direct || qc.vpart) {
+      if (direct) qc.row0 = qkv.Dq + qkv.Dkv;  // the V rows only
+      if ((rc = m->neox ? sh_qkv_finish_head_launch(e, gpart, nq, pq.part_stride, pq.ldo, nc, qkv, qc, L.q_norm,
+                                                    L.k_norm, m->eps, true)
+                        : sh_qkv_finish_launch(e, gpart, nq, pq.part_stride, pq.ldo, nc, qkv, qc)))
+        return rc;
+    }
+    if (m->call_cm1) {
+      FaArgs fa;
+      fa.layer = l; fa.N = nc; fa.col0 = 0; fa.kvlen = segs.back().kvlen; fa.mask_base = segs.front().mask_base;
+      fa.kv_cap = segs.front().kv->max_seq;
+      if ((rc = sh_fa16_launch(e, m, segs.front().kv, fa, q, nullptr, nullptr, nullptr, nullptr, bh))) return rc;
+    } else if ((rc = sh_fab_launch(e, m, fab.fl, l, q, w.attn, w.bx, w.xs, w.cs, bh))) {
+      return rc;
+    }
+    if ((rc = add_resid(L.wo, bh, "gemv_o"))) return rc;
+    if ((rc = norm_rows(L.ffn_norm, 0))) return rc;
+    if (sh_gemm16_splits(L.wgu, nc) == 1) {
+      EpiArgs sw;
+      sw.h16 = bh2; sw.ldh = m->ff;
+      if ((rc = sh_gemm16_launch(e, L.wgu, bh, m->d, nc, EPI_SWIGLU, sw, "gemv_gate_up"))) return rc;
+    } else {
+      const EpiArgs pg = part_args(L.wgu);
+      PrepArgs pr;
+      if ((rc = sh_gemm16_launch(e, L.wgu, bh, m->d, nc, EPI_PART, pg, "gemv_gate_up", &pr.nparts))) return rc;
+      pr.mode = PREP_SWIGLU; pr.part = gpart; pr.part_ld = pg.ldo; pr.part_cols = ncp; pr.K = m->ff; pr.N = nc;
+      pr.bh = bh2; pr.ldb = m->ff;
+      if ((rc = sh_prep_launch(e, pr))) return rc;
+    }
+    if ((rc = add_resid(L.wdown, bh2, "gemv_down"))) return rc;
+  }
+  if (pending && want_resid) {
+    if ((rc = sh_part_reduce_launch(e, gpart, pending, pending_ld, ncp, m->d, nc, resid, m->d, true))) return rc;
+    pending = 0;
+  }
+  if (lm0 < nc) {
+    if ((rc = norm_rows(m->out_norm, lm0))) return rc;
+    EpiArgs st;
+    st.out = w.logits; st.ldo = m->V; st.rows = m->V;
+    if ((rc = sh_gemm16_launch(e, m->lm_head, bh, m->d, nc - lm0, EPI_STORE, st, "gemv_lm_head"))) return rc;
+  }
+  return SH_OK;
+}
+
 // Columns per forward chunk: SH_MAX_COLS when the multi-group path applies
 // (all matrices K-quants) and takes the chunk (more than 8 columns, or a model
 // the fused path cannot run), else 8.
@@ -1240,8 +1408,19 @@ static uint32_t fa_seg_cols(const sh_model* m) {
   return std::max<uint32_t>(8, std::min<uint32_t>(SH_MAX_COLS, (uint32_t)SH_FA_MAX_ROWS / gqa));
 }
 
+// Runs one chunk; logits wanted of columns lm0 .. nc - 1 (nc: none). The rows
+// before lm0 may be computed as well (out->logit0: the column of w.logits row 0).
 static int run_chunk(sh_model* m, const uint32_t* dev_tokens, uint32_t nc, const ColKv* cols,
-                     const std::vector<FaSeg>& segs, bool want_logits, bool want_resid) {
+                     const std::vector<FaSeg>& segs, uint32_t lm0, bool want_resid, ChunkOut* out) {
+  const bool want_logits = lm0 < nc;
+  bool w16 = m->call16 && !m->n_expert && !cols[0].kv->graph_base;
+  if (w16 && !m->call_cm1) {
+    w16 = fab_enabled() && !(segs.size() == 1 && segs[0].ncol <= 8);
+    for (const FaSeg& sg : segs) w16 = w16 && sg.hmasks;
+  }
+  if (w16) return forward_chunk_w16(m, dev_tokens, nc, cols, segs, lm0, want_resid, out);
+  out->resid = m->ws.resid;
+  out->logit0 = 0;
   return (nc > 8 || !m->fused_ok || m->call16) ? forward_chunk_mg(m, dev_tokens, nc, cols, segs, want_logits, want_resid)
                                            : forward_chunk(m, dev_tokens, nc, cols, segs, want_logits, want_resid);
 }
@@ -1352,8 +1531,19 @@ static int forward_dev(sh_model* m, sh_kv* kv, const uint32_t* dev_tokens, uint3
   // a masked forward of more than one token: the reference's cm1 attention
   // (models/llama.rs:216-222, ops/flash_attn.rs:442-471)
   m->call_cm1 = m->fa16 && L > 1 && !parents;
-  const uint32_t CW = chunk_cols(m, L);
-  if (m->call_cm1 && !graph && (rc = ensure_fa16(m, pos + L, std::min(L, CW)))) return rc;
+  uint32_t CW = chunk_cols(m, L);
+  // a prefill (no logits, or the last column's): passes of up to SH_MAX_COLS_T
+  // columns, as even as 32-column groups allow
+  if (CW == SH_MAX_COLS16 && m->call_cm1 && m->big16_ok && logits_mode != 2 && L > SH_MAX_COLS16) {
+    const uint32_t np = (L + SH_MAX_COLS_T - 1) / SH_MAX_COLS_T;
+    CW = ((L + np - 1) / np + 31) / 32 * 32;
+  }
+  if (m->call_cm1 && !graph)
+    for (uint32_t c0 = 0; c0 < L; c0 += CW) {  // the split attention's buffers, for the chunks that take it
+      FaArgs fa;
+      fa.N = std::min(CW, L - c0); fa.kvlen = pos + c0 + fa.N;
+      if (!sh_fa16_rows(m, fa, m->call16) && (rc = ensure_fa16(m, fa.kvlen, fa.N))) return rc;
+    }
   // Attention: one segment per chunk (device masks) on the multi-group path,
   // else pieces of <= 8 columns; a causal segment's masks are relative to its
   // first column.
@@ -1396,20 +1586,22 @@ static int forward_dev(sh_model* m, sh_kv* kv, const uint32_t* dev_tokens, uint3
       cols[j].kv = kv; cols[j].slot = pos + c0 + j; cols[j].pos = plan.colpos[c0 + j];
     }
     const std::vector<FaSeg>& segs = chunk_segs[c0 / CW];
-    if ((rc = run_chunk(m, dev_tokens + c0, nc, cols.data(), segs, want, resid_host != nullptr))) return rc;
+    const uint32_t j0 = logits_mode == 1 ? nc - 1 : 0;
+    ChunkOut co;
+    if ((rc = run_chunk(m, dev_tokens + c0, nc, cols.data(), segs, want ? j0 : nc, resid_host != nullptr, &co))) return rc;
     if (resid_host)
-      SH_HIP(hipMemcpyAsync(resid_host + (size_t)c0 * m->d, m->ws.resid, (size_t)nc * m->d * 4,
-                            hipMemcpyDeviceToHost, e->stream));
+      SH_HIP(hipMemcpyAsync(resid_host + (size_t)c0 * m->d, co.resid, (size_t)nc * m->d * 4, hipMemcpyDeviceToHost,
+                            e->stream));
     if (want) {
-      const uint32_t j0 = logits_mode == 1 ? nc - 1 : 0;
       const uint32_t ncopy = nc - j0;
+      const float* lg = m->ws.logits + (size_t)(j0 - co.logit0) * m->V;
       const uint32_t dst_col = logits_mode == 1 ? 0 : c0;
       if (logits_dev_out)
-        SH_HIP(hipMemcpyAsync(logits_dev_out + (size_t)dst_col * m->V, m->ws.logits + (size_t)j0 * m->V,
-                              (size_t)ncopy * m->V * 4, hipMemcpyDeviceToDevice, e->stream));
+        SH_HIP(hipMemcpyAsync(logits_dev_out + (size_t)dst_col * m->V, lg, (size_t)ncopy * m->V * 4,
+                              hipMemcpyDeviceToDevice, e->stream));
       if (logits_host)
-        SH_HIP(hipMemcpyAsync(logits_host + (size_t)dst_col * m->V, m->ws.logits + (size_t)j0 * m->V,
-                              (size_t)ncopy * m->V * 4, hipMemcpyDeviceToHost, e->stream));
+        SH_HIP(hipMemcpyAsync(logits_host + (size_t)dst_col * m->V, lg, (size_t)ncopy * m->V * 4, hipMemcpyDeviceToHost,
+                              e->stream));
     }
     if (resid_host || logits_host) SH_HIP(hipStreamSynchronize(e->stream));
   }
@@ -1639,10 +1831,11 @@ static int verify_unified_impl(sh_engine* e, sh_model* m, sh_kv* const* caches, 
   for (uint32_t c0 = 0; c0 < N && !rc; c0 += CW) {
     const uint32_t nc = std::min<uint32_t>(CW, N - c0);
     const std::vector<FaSeg>& segs = chunk_segs[c0 / CW];
-    rc = run_chunk(m, dt + c0, nc, cols.data() + c0, segs, want_logits, residual_out != nullptr);
+    ChunkOut co;
+    rc = run_chunk(m, dt + c0, nc, cols.data() + c0, segs, want_logits ? 0 : nc, residual_out != nullptr, &co);
     if (rc) break;
     if (residual_out)
-      SH_HIP(hipMemcpyAsync(residual_out + (size_t)c0 * m->d, m->ws.resid, (size_t)nc * m->d * 4,
+      SH_HIP(hipMemcpyAsync(residual_out + (size_t)c0 * m->d, co.resid, (size_t)nc * m->d * 4,
                             hipMemcpyDeviceToHost, e->stream));
     if (logits_out)
       SH_HIP(hipMemcpyAsync(logits_out + (size_t)c0 * m->V, m->ws.logits, (size_t)nc * m->V * 4,

@@ -118,12 +118,12 @@ struct sh_engine {
   std::vector<GraphEntry> graphs;
   // Device scratch kept by the engine and reused by later calls (the engine
   // stream orders them): grown on demand by sh_engine_scratch.
-  void* scr[4] = {nullptr, nullptr, nullptr, nullptr};
-  size_t scr_bytes[4] = {0, 0, 0, 0};
+  void* scr[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
+  size_t scr_bytes[5] = {0, 0, 0, 0, 0};
   uint64_t graph_captures = 0, graph_launches = 0;  // replay counters (sh_engine_graph_stats)
 };
 // Scratch slots of sh_engine_scratch.
-enum ScratchSlot { SCR_ACCEPT = 0, SCR_UNIFORMS = 1, SCR_TREE = 2, SCR_SMALL = 3 };
+enum ScratchSlot { SCR_ACCEPT = 0, SCR_UNIFORMS = 1, SCR_TREE = 2, SCR_SMALL = 3, SCR_WIDE = 4, SCR_SLOTS = 5 };
 // *out = the engine's scratch of slot, at least `bytes` long. Growing it
 // waits for the stream (earlier launches may still read the old block).
 int sh_engine_scratch(sh_engine* e, int slot, size_t bytes, void** out);
@@ -179,6 +179,7 @@ struct Workspace {
   float* cs = nullptr;        // [max(K)/256][8] inverse activation scales of the current B operand
   float* ssq = nullptr;       // [max(K)/256][8] per-superblock sums of squares of the normalized input
   uint16_t* bh = nullptr;     // [cols][max(K)] f16 operand rows of the wide f16 GEMM
+  uint16_t* bh2 = nullptr;    // [cols][ff] the down operand's (its producer still reads bh)
   QkvColDev* qtab = nullptr;  // [cols] the chunk's QKV finish column table
   size_t fa_part_floats = 0;
   float* fab_part = nullptr;  // batched attention partials of every segment of a chunk (grown on demand)
@@ -242,6 +243,7 @@ struct sh_model {
   // routed experts, every matrix Q4_K), wide16 the switch (default on where
   // allowed), call16 set for the forward call in progress.
   bool wide16_ok = false;
+  bool big16_ok = false;  // dense, layers all Q4_K: prefill in passes of up to SH_MAX_COLS_T columns
   bool wide16 = false;
   bool call16 = false;
   // Causal single-sequence forward calls of more than one column compute
@@ -276,6 +278,7 @@ void sh_qmat_free(QMat* m);
 // GEMV epilogues. EPI_PART writes split-K partial sums in packed row order,
 // out[ks * part_stride + col * ldo + row], finished by the consumer (the next
 // prep kernel or sh_part_reduce_launch).
+struct QkvColDev;
 enum EpiKind { EPI_STORE = 0, EPI_ADD = 1, EPI_QKV = 2, EPI_SWIGLU = 3, EPI_PART = 4 };
 struct EpiArgs {
   float* out = nullptr;   // STORE/ADD: [N][ldo]; QKV: roped q [N][Dq]; SWIGLU: h [N][ldo]; PART: partials
@@ -301,6 +304,13 @@ struct EpiArgs {
   uint16_t* vc[8] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
   // Graph replay: colpos and slot are offsets from the device value *dbase.
   const uint32_t* dbase = nullptr;
+  // sh_gemm16_launch's whole-sum epilogues: QKV columns from a device table,
+  // row 0 of the matrix being row row_base of [q | k | v]; SWIGLU writes
+  // f16(silu(gate) up) to h16[col][ldh] (the down operand's rows).
+  const QkvColDev* tab = nullptr;
+  uint32_t row_base = 0;
+  uint16_t* h16 = nullptr;
+  uint32_t ldh = 0;
 };
 // Where a split-K GEMV takes its activation operand from: the staged operand
 // (B/XS/cs, the default), f32 rows x [N][ldx] (the operand is built in LDS, as
@@ -379,7 +389,8 @@ size_t sh_gemm_part_floats(const QMat& w);  // for SH_MAX_COLS columns
 // rows bh[col * ldb + k] (k_prep16_*), W Q4_K, Q5_K, Q6_K or Q8_0: EPI_PART
 // (partials as sh_gemm_launch's; *nparts = splits) or EPI_STORE (out[col][row]).
 // Where sh_gemm16_splits(w, N) is 1 the launch covers whole sums with EPI_PART
-// as well, and EPI_STORE / EPI_ADD (out[col][row] += ...) save the partials;
+// as well, and EPI_STORE, EPI_ADD (out[col][row] += ...), EPI_QKV (ea.tab) and
+// EPI_SWIGLU (ea.h16) save the partials and the launch that finishes them;
 // 0: another kernel takes the call.
 uint32_t sh_gemm16_max_cols(const QMat& w);
 uint32_t sh_gemm16_splits(const QMat& w, uint32_t N);
@@ -412,8 +423,8 @@ struct QkvColDev {  // one column of a device-resident column table
   uint16_t* vc;
 };
 struct QkvCols {  // per column: RoPE position, cache slot, capacity, K and V caches
-  // With tab set, the columns come from that device table (up to
-  // SH_MAX_COLS16 of them) and the arrays below are unused.
+  // With tab set, the columns come from that device table (any number of them)
+  // and the arrays below are unused.
   const QkvColDev* tab = nullptr;
   int32_t pos[SH_MAX_COLS];
   uint32_t slot[SH_MAX_COLS];
@@ -507,7 +518,7 @@ int sh_fa_launch(sh_engine* e, const sh_model* m, const sh_kv* kv, const FaArgs&
 // Attention of a single-sequence causal chunk (columns [col0, col0 + N) of the
 // forward chunk, keys [0, kvlen), chunk keys from mask_base) with the
 // reference's cooperative-matrix flash attention arithmetic (attn16.hip):
-// writes attn_out [N][n_head * hd] and the Wo operand (hi/lo groups bx, xs,
+// writes attn_out [N][n_head * hd] (null: not) and the Wo operand (hi/lo groups bx, xs,
 // cs, or with bh the f16 rows of the wide f16 GEMM). Graph replay as
 // sh_fa_launch (fa.dbase, fa.kv_cap).
 struct Fa16Args {
@@ -525,6 +536,9 @@ struct Fa16Args {
 };
 int sh_fa16_launch(sh_engine* e, const sh_model* m, const sh_kv* kv, const FaArgs& fa, const float* q,
                    float* attn_out, uint16_t* bx, uint16_t* xs, float* cs, uint16_t* bh = nullptr);
+// Whether that launch takes the one-pass kernel (k_fa16_rows: f16_rows = the Wo
+// operand is f16 rows), which needs none of the buffers below.
+bool sh_fa16_rows(const sh_model* m, const FaArgs& fa, bool f16_rows);
 // Buffer sizes sh_fa16_launch needs for N columns over keys [0, kv_cap).
 size_t sh_fa16_pv_halves(uint32_t n_kv, uint32_t hd, uint32_t gqa, uint32_t ncol, uint32_t kv_cap);
 size_t sh_fa16_sync_words(uint32_t n_kv, uint32_t gqa, uint32_t ncol, uint32_t kv_cap);
