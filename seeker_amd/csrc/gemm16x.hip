@@ -5,8 +5,10 @@
 // weight dequantized in f32 and rounded to f16 (stage_a_tile), each activation
 // rounded to f16, f32 accumulation; its variants cover Q8_0, Q5_K and Q6_K as
 // well as Q4_K (mmcm_variant, ops/matmul.rs:238-290). Q4_K has its own tuned
-// kernels (k_gemm16*_q4k in gemv.hip); this file serves Q8_0, Q5_K and Q6_K
-// from the same repacked tiles the f32-level kernels read, with the f32
+// kernels (k_gemm16*_q4k in gemv.hip), and calls of many columns take the
+// large-tile kernel of every format (gemm16t.h; use16t in gemv.hip draws the
+// line); this file serves the small calls of Q8_0, Q5_K and Q6_K, and Q8_0
+// matrices whose K is no multiple of 128, from the same repacked tiles the f32-level kernels read, with the f32
 // dequant of the oracle's or_dequant_row done in the same order (each product
 // and difference rounded to f32 as written) and rounded once to f16:
 //   Q8_0  f16(d * q)

@@ -2788,8 +2788,14 @@ static MgPlan plan16h(const QMat& w, bool one_split, uint32_t N) {
 // gate/up and down): there its workgroups fill the chip (gate/up at 192 columns
 // 69 -> 60 us, at 96 45 -> 39 us, down at 192 44 -> 39 us); smaller matrices at
 // 65 - 128 columns leave it half-empty 32-column groups or too few workgroups
-// (6144 x 4096 at 128 columns 24 us against 21).
+// (6144 x 4096 at 128 columns 24 us against 21). The other formats, against
+// k_gemm16x (gemm16x.hip): above 64 columns always (Q6_K 4096 x 14336 at 65 / 512
+// / 2048 columns 83 -> 34, 488 -> 91, 1910 -> 258 us), above 32 from 16 M weights
+// on (4096 x 14336 at 33 columns 57 -> 34 us, 4096 x 4096 at 33 equal; 1024 x
+// 4096 slower, 15 us against 13).
 static bool use16t(const QMat& w, uint32_t N) {
+  if (w.type != GGML_Q4_K)
+    return sh_gemm16t_ok(w) && (N > SH_MAX_COLS || (N > 32 && (uint64_t)w.tiles * 16 * w.K >= (16u << 20)));
   return N > 128 || (N > SH_MAX_COLS && (uint64_t)w.tiles * 16 * w.K >= (48u << 20));
 }
 // The others: k_gemm16w3_q4k (one pass over the weights) unless its split plan
@@ -2807,12 +2813,14 @@ static bool use16h(const QMat& w, bool one_split, uint32_t N) {
 }
 
 size_t sh_gemm16_part_floats(const QMat& w, uint32_t most) {
-  if (w.type != GGML_Q4_K) return sh_gemm16x_part_floats(w);
+  const size_t t_cols = std::max<size_t>((most + 7) / 8 * 8, std::min<size_t>(16 * ((most + 7) / 8 * 8),
+                                                                          SH_PART16_BYTES / 4 / (w.tiles * 16)));
+  if (w.type != GGML_Q4_K)
+    return std::max(sh_gemm16x_part_floats(w), sh_gemm16t_ok(w) ? t_cols * w.tiles * 16 : (size_t)0);
   if (w.K % 256) return 0;
   // split-columns of the widest partial set: k_gemm16t takes at most 16 splits
   // of SH_PART16_BYTES in all (or one split)
-  size_t cols = std::max({(size_t)plan16(w, false).KS * SH_MAX_COLS, (size_t)(most + 7) / 8 * 8,
-                          std::min<size_t>(16 * ((most + 7) / 8 * 8), SH_PART16_BYTES / 4 / (w.tiles * 16))});
+  size_t cols = std::max((size_t)plan16(w, false).KS * SH_MAX_COLS, t_cols);
   for (uint32_t N = SH_MAX_COLS + 1; N <= 128; ++N)
     if (!use16t(w, N))
       cols = std::max({cols, (size_t)plan16w(w, false, N).KS * ((N + 7) / 8 * 8),
@@ -2868,20 +2876,21 @@ static void dispatch16(sh_engine* e, const QMat& w, const uint16_t* bh, uint32_t
   }
 }
 
-uint32_t sh_gemm16_max_cols(const QMat& w) { return w.type == GGML_Q4_K ? SH_MAX_COLS_T : SH_MAX_COLS16; }
+uint32_t sh_gemm16_max_cols(const QMat& w) { return sh_gemm16t_ok(w) ? SH_MAX_COLS_T : SH_MAX_COLS16; }
 
 uint32_t sh_gemm16_splits(const QMat& w, uint32_t N) {
-  return w.type == GGML_Q4_K && use16t(w, N) ? sh_gemm16t_plan(w, false, N).KS : 0;
+  return use16t(w, N) ? sh_gemm16t_plan(w, false, N).KS : 0;
 }
 
 int sh_gemm16_launch(sh_engine* e, const QMat& w, const uint16_t* bh, uint32_t ldb, uint32_t N, EpiKind epi,
                      const EpiArgs& ea, const char* tag, uint32_t* nparts) {
-  if (w.type != GGML_Q4_K) return sh_gemm16x_launch(e, w, bh, ldb, N, epi, ea, tag, nparts);  // gemm16x.hip
+  if (w.type != GGML_Q4_K && !use16t(w, N))
+    return sh_gemm16x_launch(e, w, bh, ldb, N, epi, ea, tag, nparts);  // gemm16x.hip
   SH_CHECK(N >= 1 && N <= SH_MAX_COLS_T, SH_ERR_ARG, "f16 gemm N=%u outside [1, %u]", N, SH_MAX_COLS_T);
-  SH_CHECK(w.type == GGML_Q4_K && w.K % 256 == 0 && ldb >= w.K && ldb % 8 == 0, SH_ERR_UNSUPPORTED,
-           "f16 gemm needs Q4_K (type %d) and an operand of at least K = %u halves per column (ldb %u)", w.type, w.K,
-           ldb);
-  const bool t = use16t(w, N), one = epi != EPI_PART;
+  const bool t = use16t(w, N);
+  SH_CHECK((t || (w.type == GGML_Q4_K && w.K % 256 == 0)) && ldb >= w.K && ldb % 8 == 0, SH_ERR_UNSUPPORTED,
+           "f16 gemm: type %d, K = %u, operand of %u halves per column", w.type, w.K, ldb);
+  const bool one = epi != EPI_PART;
   SH_CHECK(epi == EPI_PART || epi == EPI_STORE || t, SH_ERR_ARG, "f16 gemm epilogue %d", (int)epi);
   const bool h = !t && N > SH_MAX_COLS && use16h(w, one, N);
   Gemm16tPlan pt;

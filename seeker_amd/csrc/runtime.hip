@@ -386,7 +386,7 @@ static int load_model(sh_engine* e, const uint8_t* img, uint64_t size, sh_model*
     m->wide16_ok = w16;
     bool big = w16 && !m->n_expert;
     for (const Layer& L : m->layers)
-      for (const QMat* q : {&L.wqkv, &L.wv, &L.wo, &L.wgu, &L.wdown}) big = big && (!q->d || q->type == GGML_Q4_K);
+      for (const QMat* q : {&L.wqkv, &L.wv, &L.wo, &L.wgu, &L.wdown}) big = big && (!q->d || sh_gemm16t_ok(*q));
     m->big16_ok = big;
     const char* env16 = getenv("SH_WIDE_F16");
     m->wide16 = w16 && !(env16 && atoi(env16) == 0);

@@ -243,7 +243,7 @@ struct sh_model {
   // routed experts, every matrix Q4_K), wide16 the switch (default on where
   // allowed), call16 set for the forward call in progress.
   bool wide16_ok = false;
-  bool big16_ok = false;  // dense, layers all Q4_K: prefill in passes of up to SH_MAX_COLS_T columns
+  bool big16_ok = false;  // dense, every layer matrix on the large-tile GEMM: prefill in passes of up to SH_MAX_COLS_T columns
   bool wide16 = false;
   bool call16 = false;
   // Causal single-sequence forward calls of more than one column compute
@@ -404,7 +404,10 @@ size_t sh_gemm16_part_floats(const QMat& w, uint32_t most = SH_MAX_COLS16);
 struct Gemm16tPlan {
   uint32_t CG = 8, ncb = 1, HS = 0, KS = 1;
 };
+bool sh_gemm16t_ok(const QMat& w);
 Gemm16tPlan sh_gemm16t_plan(const QMat& w, bool one_split, uint32_t N);
+void sh_gemm16t_fmt_launch(sh_engine* e, const QMat& w, const uint16_t* bh, uint32_t ldb, uint32_t N,
+                           const Gemm16tPlan& p, EpiKind epi, const EpiArgs& ea);  // Q5_K, Q6_K, Q8_0
 int sh_gemm16t_launch(sh_engine* e, const QMat& w, const uint16_t* bh, uint32_t ldb, uint32_t N, const Gemm16tPlan& p,
                       EpiKind epi, const EpiArgs& ea);
 // The same arithmetic for Q8_0, Q5_K and Q6_K weights (gemm16x.hip), which

@@ -106,3 +106,27 @@ def test_wide16_large_tile(engine, M, K, N, acc):
     print(f"  vs or_gemv16 {err:.2e}, vs exact {dex:.2e}", flush=True)
     assert err < 2e-5, err
     assert dex > 2 * err
+
+
+# The same edges for the formats with their own decode in the large-tile kernel
+# (Q8_0 in units of 128 k: 1408 = 11). Bound as test_wide16_other_formats.
+@pytest.mark.parametrize("qtype", [GGML_Q8_0, GGML_Q5_K, GGML_Q6_K], ids=["q8_0", "q5k", "q6k"])
+@pytest.mark.parametrize("M,K,N,acc", [(37, 256, 65, False), (512, 1408, 129, True), (4100, 512, 321, False),
+                                       (300, 768, 1025, True), (256, 4096, 257, False)])
+def test_wide16_large_tile_formats(engine, qtype, M, K, N, acc):
+    if qtype != GGML_Q8_0:
+        K = K // 256 * 256
+    print(f"wide16 {qtype} M={M} K={K} N={N} acc={acc}", flush=True)
+    w = S.quantize(qtype, S.normal_f32(M + K, 2, M * K, 0.0, 0.02))
+    rng = np.random.default_rng(N)
+    x = rng.standard_normal((N, K)).astype(np.float32)
+    y0 = rng.standard_normal((N, M)).astype(np.float32) if acc else np.zeros((N, M), np.float32)
+    qt = QTensor(engine, qtype, w, M, K)
+    xd, yd = engine.to_device(x), engine.to_device(y0)
+    engine.gemm_wide16(qt, xd, N, yd, acc)
+    got = yd.read(np.float32, N * M).reshape(N, M)
+    ref = O.gemv16(qtype, w, M, K, x) + (y0 if acc else 0)
+    xd.free(); yd.free(); qt.close()
+    err = np.abs(got - ref).max() / np.abs(ref).max()
+    print(f"  vs or_gemv16 {err:.2e}", flush=True)
+    assert err < 1e-5, err
