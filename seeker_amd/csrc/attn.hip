@@ -675,15 +675,12 @@ __global__ void k_kv_scatter(uint16_t* __restrict__ k, uint16_t* __restrict__ v,
   vh[((size_t)(s / 32) * hd + d) * 32 + v_slot_a(s & 31)] = st[hd + d];
 }
 
-int sh_kv_compact_launch(sh_engine* e, sh_kv* kv, uint32_t base, const uint32_t* src_dev, uint32_t n) {
+int sh_kv_compact_launch(sh_engine* e, sh_kv* kv, uint32_t base, const uint32_t* src_dev, uint32_t n, uint16_t* stage) {
   const uint32_t lh = kv->n_layer * kv->n_kv;
-  uint16_t* stage = nullptr;
-  SH_HIP(hipMallocAsync((void**)&stage, (size_t)lh * n * kv->hd * 2 * 2, e->stream));
   hipLaunchKernelGGL(k_kv_gather, dim3(lh, n), dim3(kv->hd), 0, e->stream, kv->k, kv->v, stage, kv->max_seq, kv->hd,
                      base, src_dev, n);
   hipLaunchKernelGGL(k_kv_scatter, dim3(lh, n), dim3(kv->hd), 0, e->stream, kv->k, kv->v, stage, kv->max_seq,
                      kv->hd, base, n);
   SH_HIP(hipGetLastError());
-  SH_HIP(hipFreeAsync(stage, e->stream));
   return SH_OK;
 }

@@ -491,7 +491,9 @@ int sh_fab_plan(sh_engine* e, sh_model* m, const FabSegIn* in, uint32_t nseg, ui
       hm[in[s].col0 + j] = in[s].hmasks[j];
     }
   }
-  SH_HIP(hipMallocAsync((void**)&out->dev, bytes, e->stream));
+  void* dev = nullptr;
+  if (int rc = sh_engine_scratch(e, SCR_FAB, bytes, &dev)) return rc;
+  out->dev = (uint8_t*)dev;
   for (uint32_t s = 0; s < nseg; ++s) segs[s].masks = (const uint64_t*)(out->dev + o_mask) + in[s].col0;
   std::memcpy(host.data(), segs.data(), nseg * sizeof(FabSeg));
   std::memcpy(host.data() + o_work, work.data(), work.size() * 4);
@@ -513,11 +515,6 @@ int sh_fab_plan(sh_engine* e, sh_model* m, const FabSegIn* in, uint32_t nseg, ui
   }
   out->part = w.fab_part;
   return SH_OK;
-}
-
-void sh_fab_free(sh_engine* e, FabLaunch& fl) {
-  if (fl.dev) (void)hipFreeAsync(fl.dev, e->stream);
-  fl.dev = nullptr;
 }
 
 int sh_fab_launch(sh_engine* e, const sh_model* m, const FabLaunch& fl, uint32_t layer, const float* q, float* attn_out,

@@ -164,13 +164,17 @@ extern "C" int sh_engine_profile_reset(sh_engine* e) {
 int sh_engine_scratch(sh_engine* e, int slot, size_t bytes, void** out) {
   SH_CHECK(slot >= 0 && slot < SCR_SLOTS, SH_ERR_ARG, "scratch slot %d", slot);
   if (bytes > e->scr_bytes[slot]) {
-    g_graph_gen.fetch_add(1);  // captured graphs may point into the old block
+    if (slot < SCR_WIDE) g_graph_gen.fetch_add(1);  // captured graphs may point into the old block
     SH_HIP(hipStreamSynchronize(e->stream));
+    const size_t old = e->scr_bytes[slot];
     if (e->scr[slot]) SH_HIP(hipFree(e->scr[slot]));
     e->scr[slot] = nullptr;
     e->scr_bytes[slot] = 0;
-    const size_t cap = (bytes + 4095) / 4096 * 4096;
+    size_t cap = (bytes + 4095) / 4096 * 4096;
+    if (slot >= SCR_WIDE)  // sizes vary from call to call: grow by a quarter at least
+      cap = std::max(cap, (old + old / 4 + 4095) / 4096 * 4096);
     SH_HIP(hipMalloc(&e->scr[slot], cap));
+    if (slot == SCR_XS) SH_HIP(hipMemsetAsync(e->scr[slot], 0, cap, e->stream));
     e->scr_bytes[slot] = cap;
   }
   *out = e->scr[slot];
@@ -599,12 +603,14 @@ extern "C" int sh_kv_compact(sh_kv* kv, uint32_t base, const uint32_t* src, uint
     SH_CHECK(base + src[i] < kv->max_seq, SH_ERR_ARG, "compaction source %u out of range", src[i]);
   if (n) {
     sh_engine* e = kv->e;
-    uint32_t* d = nullptr;
-    SH_HIP(hipMallocAsync((void**)&d, n * 4, e->stream));
-    SH_HIP(hipMemcpyAsync(d, src, n * 4, hipMemcpyHostToDevice, e->stream));
-    int rc = sh_kv_compact_launch(e, kv, base, d, n);
+    ScratchLayout lay;
+    const size_t o_src = lay.take((size_t)n * 4), o_stage = lay.take((size_t)kv->n_layer * kv->n_kv * n * kv->hd * 4);
+    void* d = nullptr;
+    int rc = sh_engine_scratch(e, SCR_COLS, lay.bytes, &d);
     if (rc) return rc;
-    SH_HIP(hipFreeAsync(d, e->stream));
+    uint32_t* src_dev = (uint32_t*)((uint8_t*)d + o_src);
+    SH_HIP(hipMemcpyAsync(src_dev, src, n * 4, hipMemcpyHostToDevice, e->stream));
+    if ((rc = sh_kv_compact_launch(e, kv, base, src_dev, n, (uint16_t*)((uint8_t*)d + o_stage)))) return rc;
     SH_HIP(hipStreamSynchronize(e->stream));
   }
   kv->pos = base + n;
@@ -654,20 +660,14 @@ static bool fab_enabled() {
   return v;
 }
 
-struct FabGuard {  // a chunk's batched-attention plan, freed (stream-ordered) at scope end
-  sh_engine* e;
-  FabLaunch fl;
-  ~FabGuard() { sh_fab_free(e, fl); }
-};
-
-static int plan_fab(sh_model* m, const std::vector<FaSeg>& segs, uint32_t nc, FabGuard* g) {
+static int plan_fab(sh_model* m, const std::vector<FaSeg>& segs, uint32_t nc, FabLaunch* fl) {
   std::vector<FabSegIn> fin(segs.size());
   for (size_t i = 0; i < segs.size(); ++i) {
     const FaSeg& sg = segs[i];
     fin[i].kv = sg.kv; fin[i].col0 = sg.col0; fin[i].ncol = sg.ncol; fin[i].kvlen = sg.kvlen;
     fin[i].mask_base = sg.mask_base; fin[i].hmasks = sg.hmasks;
   }
-  return sh_fab_plan(m->e, m, fin.data(), (uint32_t)fin.size(), nc, &g->fl);
+  return sh_fab_plan(m->e, m, fin.data(), (uint32_t)fin.size(), nc, fl);
 }
 
 // SH_FUSE=0 keeps the separate down prep and attention combine kernels.
@@ -1099,7 +1099,7 @@ static int forward_chunk_mg(sh_model* m, const uint32_t* dev_tokens, uint32_t nc
   const bool cm1 = m->call_cm1;
   SH_CHECK(!cm1 || (segs.front().col0 == 0 && segs.back().col0 + segs.back().ncol == nc), SH_ERR_ARG,
            "cm1 attention: the segments must cover the chunk");
-  FabGuard fab{e, FabLaunch{}};
+  FabLaunch fab;
   // one sequence's chain of at most 8 columns (the draft's forwards, graph
   // captures) takes the split attention with its masks as kernel arguments
   const bool single8 = segs.size() == 1 && segs[0].ncol <= 8;
@@ -1139,7 +1139,7 @@ static int forward_chunk_mg(sh_model* m, const uint32_t* dev_tokens, uint32_t nc
       if ((rc = sh_fa16_launch(e, m, segs.front().kv, fa, w.q, w.attn, w.bx, w.xs, w.cs, f16 ? w.bh : nullptr)))
         return rc;
     } else if (use_fab) {
-      if ((rc = sh_fab_launch(e, m, fab.fl, l, w.q, w.attn, w.bx, w.xs, w.cs, f16 ? w.bh : nullptr))) return rc;
+      if ((rc = sh_fab_launch(e, m, fab, l, w.q, w.attn, w.bx, w.xs, w.cs, f16 ? w.bh : nullptr))) return rc;
     } else {
       for (const FaSeg& sg : segs) {
         FaArgs fa;
@@ -1255,17 +1255,12 @@ static int forward_chunk_w16(sh_model* m, const uint32_t* dev_tokens, uint32_t n
     while (C < nc) C *= 2;
     gpart_floats = 0;
     for (const Layer& L : m->layers) gpart_floats = std::max(gpart_floats, layer_part16_floats(L, C));
-    size_t off = 0;
-    auto take = [&](size_t bytes) {
-      const size_t o = off;
-      off += (bytes + 255) / 256 * 256;
-      return o;
-    };
-    const size_t o_resid = take((size_t)C * m->d * 4), o_q = take((size_t)C * wide * 4), o_bh = take((size_t)C * wide * 2),
-                 o_bh2 = take((size_t)C * m->ff * 2), o_tab = take((size_t)C * sizeof(QkvColDev)),
-                 o_part = take(gpart_floats * 4);
+    ScratchLayout lay;
+    const size_t o_resid = lay.take((size_t)C * m->d * 4), o_q = lay.take((size_t)C * wide * 4),
+                 o_bh = lay.take((size_t)C * wide * 2), o_bh2 = lay.take((size_t)C * m->ff * 2),
+                 o_tab = lay.take((size_t)C * sizeof(QkvColDev)), o_part = lay.take(gpart_floats * 4);
     void* base = nullptr;
-    if ((rc = sh_engine_scratch(e, SCR_WIDE, off, &base))) return rc;
+    if ((rc = sh_engine_scratch(e, SCR_WIDE, lay.bytes, &base))) return rc;
     uint8_t* b = (uint8_t*)base;
     resid = (float*)(b + o_resid); q = (float*)(b + o_q); bh = (uint16_t*)(b + o_bh); bh2 = (uint16_t*)(b + o_bh2);
     qtab = (QkvColDev*)(b + o_tab); gpart = (float*)(b + o_part);
@@ -1311,7 +1306,7 @@ static int forward_chunk_w16(sh_model* m, const uint32_t* dev_tokens, uint32_t n
     pending_ld = pa.ldo;
     return sh_gemm16_launch(e, mat, rows, mat.K, nc, EPI_PART, pa, tag, &pending);
   };
-  FabGuard fab{e, FabLaunch{}};
+  FabLaunch fab;
   if (!m->call_cm1 && (rc = plan_fab(m, segs, nc, &fab))) return rc;
   const bool rope4 = !m->neox && qkv.Dq % 64 == 0 && qkv.Dkv % 64 == 0;
   for (uint32_t l = 0; l < m->n_layer; ++l) {
@@ -1350,7 +1345,7 @@ static int forward_chunk_w16(sh_model* m, const uint32_t* dev_tokens, uint32_t n
       fa.layer = l; fa.N = nc; fa.col0 = 0; fa.kvlen = segs.back().kvlen; fa.mask_base = segs.front().mask_base;
       fa.kv_cap = segs.front().kv->max_seq;
       if ((rc = sh_fa16_launch(e, m, segs.front().kv, fa, q, nullptr, nullptr, nullptr, nullptr, bh))) return rc;
-    } else if ((rc = sh_fab_launch(e, m, fab.fl, l, q, w.attn, w.bx, w.xs, w.cs, bh))) {
+    } else if ((rc = sh_fab_launch(e, m, fab, l, q, w.attn, w.bx, w.xs, w.cs, bh))) {
       return rc;
     }
     if ((rc = add_resid(L.wo, bh, "gemv_o"))) return rc;
@@ -1506,7 +1501,7 @@ static int ensure_fa16(sh_model* m, uint32_t kv_cap, uint32_t ncol) {
 // logits_dst != null, copies logits of the selected columns there (device).
 static int forward_dev(sh_model* m, sh_kv* kv, const uint32_t* dev_tokens, uint32_t L, uint32_t pos,
                        const int32_t* parents, int logits_mode, float* logits_dev_out, float* resid_host,
-                       float* logits_host) {
+                       float* logits_host, uint64_t* dmask = nullptr) {
   sh_engine* e = m->e;
   SH_CHECK(L >= 1, SH_ERR_ARG, "empty prompt");
   const bool graph = kv->graph_base != nullptr;  // pos is an offset from *graph_base at replay
@@ -1566,17 +1561,12 @@ static int forward_dev(sh_model* m, sh_kv* kv, const uint32_t* dev_tokens, uint3
     }
     chunk_segs.push_back(segs);
   }
-  uint64_t* dmask = nullptr;
   if (CW > 8 && !m->call_cm1 && L > 8) {  // <= 8 columns: one segment, masks as kernel arguments
-    SH_HIP(hipMallocAsync((void**)&dmask, (size_t)L * 8, e->stream));
+    SH_CHECK(dmask, SH_ERR_STATE, "forward: no mask buffer");
     SH_HIP(hipMemcpyAsync(dmask, hmask.data(), (size_t)L * 8, hipMemcpyHostToDevice, e->stream));
     for (size_t c = 0; c < chunk_segs.size(); ++c)
       for (FaSeg& sg : chunk_segs[c]) sg.masks = dmask + c * CW + sg.col0;
   }
-  struct MaskFree {  // the masks stay allocated until every launch that reads them is queued
-    sh_engine* e; uint64_t* p;
-    ~MaskFree() { if (p) (void)hipFreeAsync(p, e->stream); }
-  } mask_free{e, dmask};
   for (uint32_t c0 = 0; c0 < L; c0 += CW) {
     const uint32_t nc = std::min<uint32_t>(CW, L - c0);
     const bool last = c0 + nc == L;
@@ -1609,14 +1599,25 @@ static int forward_dev(sh_model* m, sh_kv* kv, const uint32_t* dev_tokens, uint3
   return SH_OK;
 }
 
-static int upload_tokens(sh_model* m, const uint32_t* tokens, uint32_t L, uint32_t** dev) {
-  uint32_t* d = nullptr;
+// A forward call's device columns: token ids (uploaded), room for a mask and a
+// sampled id per column, in the engine's scratch.
+struct DevCols {
+  uint32_t* tokens = nullptr;
+  uint64_t* masks = nullptr;
+  uint32_t* ids = nullptr;
+};
+static int upload_tokens(sh_model* m, const uint32_t* tokens, uint32_t L, DevCols* dev) {
   SH_CHECK(tokens, SH_ERR_ARG, "tokens is NULL");
   for (uint32_t i = 0; i < L; ++i)
     SH_CHECK(tokens[i] < m->V, SH_ERR_ARG, "token id %u out of range (vocab %u)", tokens[i], m->V);
-  SH_HIP(hipMalloc(&d, (size_t)L * 4));
-  SH_HIP(hipMemcpyAsync(d, tokens, (size_t)L * 4, hipMemcpyHostToDevice, m->e->stream));
-  *dev = d;
+  ScratchLayout lay;
+  const size_t o_tok = lay.take((size_t)L * 4), o_mask = lay.take((size_t)L * 8), o_ids = lay.take((size_t)L * 4);
+  void* base = nullptr;
+  if (int rc = sh_engine_scratch(m->e, SCR_COLS, lay.bytes, &base)) return rc;
+  dev->tokens = (uint32_t*)((uint8_t*)base + o_tok);
+  dev->masks = (uint64_t*)((uint8_t*)base + o_mask);
+  dev->ids = (uint32_t*)((uint8_t*)base + o_ids);
+  SH_HIP(hipMemcpyAsync(dev->tokens, tokens, (size_t)L * 4, hipMemcpyHostToDevice, m->e->stream));
   return SH_OK;
 }
 
@@ -1626,13 +1627,12 @@ extern "C" int sh_forward_full(sh_engine* e, sh_model* m, sh_kv* kv, const uint3
   SH_CHECK(e && m && kv, SH_ERR_ARG, "sh_forward_full: NULL handle");
   SH_CHECK(logits_mode >= 0 && logits_mode <= 2, SH_ERR_ARG, "logits_mode %d", logits_mode);
   SH_CHECK(L >= 1, SH_ERR_ARG, "empty prompt");
-  uint32_t* dt = nullptr;
-  int rc = upload_tokens(m, tokens, L, &dt);
+  DevCols dc;
+  int rc = upload_tokens(m, tokens, L, &dc);
   if (rc) return rc;
-  rc = forward_dev(m, kv, dt, L, pos, parents, logits_mode, nullptr, residual_out,
-                   logits_mode ? logits_out : nullptr);
+  rc = forward_dev(m, kv, dc.tokens, L, pos, parents, logits_mode, nullptr, residual_out,
+                   logits_mode ? logits_out : nullptr, dc.masks);
   hipError_t se = hipStreamSynchronize(e->stream);
-  (void)hipFree(dt);
   if (rc) return rc;
   SH_CHECK(se == hipSuccess, SH_ERR_HIP, "forward: %s", hipGetErrorString(se));
   kv->pending.clear();
@@ -1700,23 +1700,19 @@ extern "C" int sh_verify_greedy(sh_engine* e, sh_model* m, sh_kv* kv, const uint
              "KV cache dims do not match the model");
     return verify_greedy_graph(e, m, kv, tokens, L, pos, sampled_out);
   }
-  uint32_t* dt = nullptr;
-  int rc = upload_tokens(m, tokens, L, &dt);
+  DevCols dc;
+  int rc = upload_tokens(m, tokens, L, &dc);
   if (rc) return rc;
-  float* lg = nullptr;
-  SH_HIP(hipMallocAsync((void**)&lg, (size_t)L * m->V * 4, e->stream));
-  uint32_t* ids = nullptr;
-  SH_HIP(hipMallocAsync((void**)&ids, 64 * 4, e->stream));
-  rc = forward_dev(m, kv, dt, L, pos, nullptr, 2, lg, nullptr, nullptr);
-  if (!rc) rc = sh_argmax_launch(e, lg, m->V, L, m->ws.amax, ids);
+  void* lgv = nullptr;
+  if ((rc = sh_engine_scratch(e, SCR_VERIFY, (size_t)L * m->V * 4, &lgv))) return rc;
+  float* lg = (float*)lgv;
+  rc = forward_dev(m, kv, dc.tokens, L, pos, nullptr, 2, lg, nullptr, nullptr, dc.masks);
+  if (!rc) rc = sh_argmax_launch(e, lg, m->V, L, m->ws.amax, dc.ids);
   if (!rc) {
-    hipError_t ce = hipMemcpyAsync(sampled_out, ids, (size_t)L * 4, hipMemcpyDeviceToHost, e->stream);
+    hipError_t ce = hipMemcpyAsync(sampled_out, dc.ids, (size_t)L * 4, hipMemcpyDeviceToHost, e->stream);
     if (ce != hipSuccess) { sh_set_error("verify readback: %s", hipGetErrorString(ce)); rc = SH_ERR_HIP; }
   }
   hipError_t se = hipStreamSynchronize(e->stream);
-  (void)hipFree(dt);
-  (void)hipFreeAsync(lg, e->stream);
-  (void)hipFreeAsync(ids, e->stream);
   if (rc) return rc;
   SH_CHECK(se == hipSuccess, SH_ERR_HIP, "verify: %s", hipGetErrorString(se));
   kv->pending.clear();
@@ -1787,10 +1783,8 @@ static int verify_unified_impl(sh_engine* e, sh_model* m, sh_kv* const* caches, 
       cols[j].kv = caches[s]; cols[j].slot = caches[s]->pos + i; cols[j].pos = plans[s].colpos[i];
       cseq[j] = s; cidx[j] = i;
     }
-  uint32_t* dt = nullptr;
-  if ((rc = upload_tokens(m, tokens, N, &dt))) return rc;
-  uint32_t* ids = nullptr;
-  if (sampled_out) SH_HIP(hipMallocAsync((void**)&ids, SH_MAX_COLS16 * 4, e->stream));
+  DevCols dc;
+  if ((rc = upload_tokens(m, tokens, N, &dc))) return rc;
   const bool want_logits = logits_out || logits_dev || sampled_out;
   m->call16 = m->wide16 && N >= SH_WIDE16_COLS;  // the reference's batch is one matmul of N columns
   m->call_cm1 = false;  // the batched attention is the reference's scalar kernel (ops/flash_attn.rs:819-1016)
@@ -1821,9 +1815,8 @@ static int verify_unified_impl(sh_engine* e, sh_model* m, sh_kv* const* caches, 
     }
     chunk_segs.push_back(segs);
   }
-  uint64_t* dmask = nullptr;
   if (CW > 8) {
-    SH_HIP(hipMallocAsync((void**)&dmask, (size_t)N * 8, e->stream));
+    uint64_t* dmask = dc.masks;
     SH_HIP(hipMemcpyAsync(dmask, hmask.data(), (size_t)N * 8, hipMemcpyHostToDevice, e->stream));
     for (size_t c = 0; c < chunk_segs.size(); ++c)
       for (FaSeg& sg : chunk_segs[c]) sg.masks = dmask + c * CW + sg.col0;
@@ -1832,7 +1825,7 @@ static int verify_unified_impl(sh_engine* e, sh_model* m, sh_kv* const* caches, 
     const uint32_t nc = std::min<uint32_t>(CW, N - c0);
     const std::vector<FaSeg>& segs = chunk_segs[c0 / CW];
     ChunkOut co;
-    rc = run_chunk(m, dt + c0, nc, cols.data() + c0, segs, want_logits ? 0 : nc, residual_out != nullptr, &co);
+    rc = run_chunk(m, dc.tokens + c0, nc, cols.data() + c0, segs, want_logits ? 0 : nc, residual_out != nullptr, &co);
     if (rc) break;
     if (residual_out)
       SH_HIP(hipMemcpyAsync(residual_out + (size_t)c0 * m->d, co.resid, (size_t)nc * m->d * 4,
@@ -1844,6 +1837,7 @@ static int verify_unified_impl(sh_engine* e, sh_model* m, sh_kv* const* caches, 
       SH_HIP(hipMemcpyAsync(logits_dev + (size_t)c0 * m->V, m->ws.logits, (size_t)nc * m->V * 4,
                             hipMemcpyDeviceToDevice, e->stream));
     if (sampled_out) {
+      uint32_t* ids = dc.ids + c0;
       if ((rc = sh_argmax_launch(e, m->ws.logits, m->V, nc, m->ws.amax, ids))) break;
       if (any_stoch) {
         // column c of sequence s (its j-th): uniform j of s's explicit array,
@@ -1866,14 +1860,14 @@ static int verify_unified_impl(sh_engine* e, sh_model* m, sh_kv* const* caches, 
           chunk_filt = chunk_filt || (!r.greedy && r.top_k);
         }
         if (chunk_plain || chunk_filt) {
-          SampRow* rdev = nullptr;
-          double2* part = nullptr;
-          SH_HIP(hipMallocAsync((void**)&rdev, nc * sizeof(SampRow), e->stream));
-          SH_HIP(hipMallocAsync((void**)&part, sh_sample_rows_part_bytes(nc, m->V), e->stream));
+          ScratchLayout lay;
+          const size_t o_row = lay.take(nc * sizeof(SampRow)), o_part = lay.take(sh_sample_rows_part_bytes(nc, m->V));
+          void* base = nullptr;
+          if ((rc = sh_engine_scratch(e, SCR_ROWS, lay.bytes, &base))) break;
+          SampRow* rdev = (SampRow*)((uint8_t*)base + o_row);
+          double2* part = (double2*)((uint8_t*)base + o_part);
           SH_HIP(hipMemcpyAsync(rdev, rows.data(), nc * sizeof(SampRow), hipMemcpyHostToDevice, e->stream));
           rc = sh_sample_rows_tab_launch(e, m->ws.logits, nc, m->V, rdev, part, ids, chunk_plain, chunk_filt);
-          (void)hipFreeAsync(rdev, e->stream);
-          (void)hipFreeAsync(part, e->stream);
           if (rc) break;
         }
       }
@@ -1881,9 +1875,6 @@ static int verify_unified_impl(sh_engine* e, sh_model* m, sh_kv* const* caches, 
     }
   }
   hipError_t se = hipStreamSynchronize(e->stream);
-  (void)hipFree(dt);
-  if (ids) (void)hipFree(ids);
-  if (dmask) (void)hipFree(dmask);
   if (rc) return rc;
   SH_CHECK(se == hipSuccess, SH_ERR_HIP, "verify_unified: %s", hipGetErrorString(se));
   for (uint32_t s = 0; s < B; ++s) {
@@ -1923,20 +1914,21 @@ extern "C" int sh_tree_verify_step(sh_engine* e, sh_model* target, sh_kv* const*
     SH_CHECK(caches[b], SH_ERR_ARG, "tree_verify_step: cache %u is NULL", b);
     base[b] = caches[b]->pos;
   }
-  float* lg = nullptr;
-  uint32_t *dtok = nullptr, *dpath = nullptr, *dlen = nullptr, *dnext = nullptr;
-  int32_t* dpar = nullptr;
-  SH_HIP(hipMallocAsync((void**)&lg, (size_t)B * n * V * 4, e->stream));
-  int rc = verify_unified_impl(e, target, caches, B, tokens, lens.data(), nullptr, parents, nullptr, lg, nullptr,
-                               nullptr);
+  ScratchLayout lay;
+  const size_t nn = (size_t)B * n * 4, o_lg = lay.take(nn * V), o_tok = lay.take(nn), o_par = lay.take(nn),
+               o_path = lay.take(nn), o_len = lay.take((size_t)B * 4), o_next = lay.take((size_t)B * 4);
+  void* base_dev = nullptr;
+  int rc = sh_engine_scratch(e, SCR_VERIFY, lay.bytes, &base_dev);
+  if (rc) return rc;
+  uint8_t* bd = (uint8_t*)base_dev;
+  float* lg = (float*)(bd + o_lg);
+  uint32_t *dtok = (uint32_t*)(bd + o_tok), *dpath = (uint32_t*)(bd + o_path), *dlen = (uint32_t*)(bd + o_len),
+           *dnext = (uint32_t*)(bd + o_next);
+  int32_t* dpar = (int32_t*)(bd + o_par);
+  rc = verify_unified_impl(e, target, caches, B, tokens, lens.data(), nullptr, parents, nullptr, lg, nullptr, nullptr);
   if (!rc) {
-    hipError_t me = hipMallocAsync((void**)&dtok, (size_t)B * n * 4, e->stream);
-    if (me == hipSuccess) me = hipMallocAsync((void**)&dpar, (size_t)B * n * 4, e->stream);
-    if (me == hipSuccess) me = hipMallocAsync((void**)&dpath, (size_t)B * n * 4, e->stream);
-    if (me == hipSuccess) me = hipMallocAsync((void**)&dlen, (size_t)B * 4, e->stream);
-    if (me == hipSuccess) me = hipMallocAsync((void**)&dnext, (size_t)B * 4, e->stream);
-    if (me == hipSuccess) me = hipMemcpyAsync(dtok, tokens, (size_t)B * n * 4, hipMemcpyHostToDevice, e->stream);
-    if (me == hipSuccess) me = hipMemcpyAsync(dpar, parents, (size_t)B * n * 4, hipMemcpyHostToDevice, e->stream);
+    hipError_t me = hipMemcpyAsync(dtok, tokens, nn, hipMemcpyHostToDevice, e->stream);
+    if (me == hipSuccess) me = hipMemcpyAsync(dpar, parents, nn, hipMemcpyHostToDevice, e->stream);
     if (me != hipSuccess) { sh_set_error("tree_verify_step: %s", hipGetErrorString(me)); rc = SH_ERR_HIP; }
   }
   if (!rc) rc = sh_tree_accept(e, lg, q_logits_dev, dtok, dpar, B, n, V, s, dpath, dlen, dnext);
@@ -1947,12 +1939,6 @@ extern "C" int sh_tree_verify_step(sh_engine* e, sh_model* target, sh_kv* const*
     if (me == hipSuccess) me = hipStreamSynchronize(e->stream);
     if (me != hipSuccess) { sh_set_error("tree_verify_step readback: %s", hipGetErrorString(me)); rc = SH_ERR_HIP; }
   }
-  (void)hipFreeAsync(lg, e->stream);
-  if (dtok) (void)hipFreeAsync(dtok, e->stream);
-  if (dpar) (void)hipFreeAsync(dpar, e->stream);
-  if (dpath) (void)hipFreeAsync(dpath, e->stream);
-  if (dlen) (void)hipFreeAsync(dlen, e->stream);
-  if (dnext) (void)hipFreeAsync(dnext, e->stream);
   if (rc) return rc;
   // keep the accepted path's K/V rows: node path[i] -> slot base + i
   for (uint32_t b = 0; b < B && !rc; ++b)
@@ -2452,20 +2438,21 @@ extern "C" int sh_gemv_quant(sh_engine* e, const sh_qtensor* w, const float* x_d
   SH_CHECK(e && w && x_dev && y_dev, SH_ERR_ARG, "sh_gemv_quant: NULL argument");
   SH_CHECK(N >= 1, SH_ERR_ARG, "N must be >= 1");
   const uint32_t K = w->m.K, M = w->m.M;
-  uint16_t *bx = nullptr, *xs = nullptr;
-  float *cs = nullptr, *part = nullptr;
   // Q4_K with more than 8 columns, and Q5_K / Q6_K at any width: the forward's
   // multi-group kernel, 64 columns per pass
   const bool mg = sh_is_kquant(w->m.type) && K % 256 == 0 && (N > 8 || w->m.type != GGML_Q4_K);
   const uint32_t CW = mg ? SH_MAX_COLS : 8, ngrp = CW / 8;
   const size_t bx_elems = ngrp * sh_grp_bx(K), xs_elems = ngrp * sh_grp_xs(K);
   const size_t part_floats = mg ? sh_gemm_part_floats(w->m) : sh_gemv_part_floats(w->m);
-  SH_HIP(hipMallocAsync((void**)&bx, bx_elems * 2, e->stream));
-  SH_HIP(hipMallocAsync((void**)&xs, xs_elems * 2, e->stream));
-  SH_HIP(hipMallocAsync((void**)&cs, ngrp * sh_grp_cs(K) * sizeof(float), e->stream));
-  SH_HIP(hipMallocAsync((void**)&part, std::max<size_t>(part_floats, 4) * sizeof(float), e->stream));
-  SH_HIP(hipMemsetAsync(xs, 0, xs_elems * 2, e->stream));
-  int rc = SH_OK;
+  ScratchLayout lay;
+  const size_t o_bx = lay.take(bx_elems * 2), o_cs = lay.take(ngrp * sh_grp_cs(K) * sizeof(float)),
+               o_part = lay.take(std::max<size_t>(part_floats, 4) * sizeof(float));
+  void *base = nullptr, *xs_base = nullptr;
+  int rc = sh_engine_scratch(e, SCR_GEMV, lay.bytes, &base);
+  if (!rc) rc = sh_engine_scratch(e, SCR_XS, xs_elems * 2, &xs_base);
+  if (rc) return rc;
+  uint16_t *bx = (uint16_t*)((uint8_t*)base + o_bx), *xs = (uint16_t*)xs_base;
+  float *cs = (float*)((uint8_t*)base + o_cs), *part = (float*)((uint8_t*)base + o_part);
   // The same kernels as the forward: split partials (finished here by a reduce)
   // where the forward would use them, else a direct store / accumulate.
   const bool split = w->m.type == GGML_Q4_K && part_floats > (size_t)8 * w->m.tiles * 16;
@@ -2504,10 +2491,6 @@ extern "C" int sh_gemv_quant(sh_engine* e, const sh_qtensor* w, const float* x_d
       rc = sh_gemv_launch(e, w->m, bx, xs, nc, accumulate ? EPI_ADD : EPI_STORE, ea, "gemv");
     }
   }
-  (void)hipFreeAsync(bx, e->stream);
-  (void)hipFreeAsync(xs, e->stream);
-  (void)hipFreeAsync(cs, e->stream);
-  (void)hipFreeAsync(part, e->stream);
   if (rc) return rc;
   SH_HIP(hipStreamSynchronize(e->stream));
   return sh_prof_flush(e);
@@ -2524,11 +2507,13 @@ extern "C" int sh_gemm_wide16(sh_engine* e, const sh_qtensor* w, const float* x_
   const uint32_t K = w->m.K, M = w->m.M, most = sh_gemm16_max_cols(w->m), npass = (N + most - 1) / most;
   const uint32_t CW = std::min(most, ((N + npass - 1) / npass + 31) / 32 * 32);
   const size_t part_floats = sh_gemm16_part_floats(w->m, CW);
-  uint16_t* bh = nullptr;
-  float* part = nullptr;
-  SH_HIP(hipMallocAsync((void**)&bh, (size_t)CW * K * 2, e->stream));
-  SH_HIP(hipMallocAsync((void**)&part, std::max<size_t>(part_floats, 4) * sizeof(float), e->stream));
-  int rc = SH_OK;
+  ScratchLayout lay;
+  const size_t o_bh = lay.take((size_t)CW * K * 2), o_part = lay.take(std::max<size_t>(part_floats, 4) * sizeof(float));
+  void* base = nullptr;
+  int rc = sh_engine_scratch(e, SCR_GEMV, lay.bytes, &base);
+  if (rc) return rc;
+  uint16_t* bh = (uint16_t*)((uint8_t*)base + o_bh);
+  float* part = (float*)((uint8_t*)base + o_part);
   for (uint32_t c0 = 0; c0 < N && !rc; c0 += CW) {
     const uint32_t nc = std::min<uint32_t>(CW, N - c0), ncp = (nc + 7) / 8 * 8;
     PrepArgs pr;
@@ -2549,8 +2534,6 @@ extern "C" int sh_gemm_wide16(sh_engine* e, const sh_qtensor* w, const float* x_
     rc = sh_gemm16_launch(e, w->m, bh, K, nc, EPI_PART, pa, "gemm16", &np);
     if (!rc) rc = sh_part_reduce_launch(e, part, np, pa.ldo, ncp, M, nc, y_dev + (size_t)c0 * M, M, accumulate != 0);
   }
-  (void)hipFreeAsync(bh, e->stream);
-  (void)hipFreeAsync(part, e->stream);
   if (rc) return rc;
   SH_HIP(hipStreamSynchronize(e->stream));
   return sh_prof_flush(e);

@@ -1458,10 +1458,10 @@ extern "C" int sh_tree_accept(sh_engine* e, const float* p_logits_dev, const flo
                "tree_accept: tree %u node %u parent %d must precede it", b, i, par[(size_t)b * n + i]);
   }
   float* udev = nullptr;
-  double* r = nullptr;
+  double* const r = nullptr;
   if (s->uniforms) {
     const size_t nu = (size_t)B * n * 2;
-    SH_HIP(hipMallocAsync((void**)&udev, nu * 4, e->stream));
+    if (int rc = sh_engine_scratch(e, SCR_UNIFORMS, nu * 4, (void**)&udev)) return rc;
     SH_HIP(hipMemcpyAsync(udev, s->uniforms, nu * 4, hipMemcpyHostToDevice, e->stream));
   }
   hipEvent_t ev = nullptr;
@@ -1489,8 +1489,9 @@ extern "C" int sh_tree_accept(sh_engine* e, const float* p_logits_dev, const flo
     const uint32_t nch = (V + 256 * kStatE - 1) / (256 * kStatE), nrows = 2 * B * n;
     const uint64_t ctr = udev ? 0ull : s->counter;
     const size_t part_b = (size_t)nrows * nch * sizeof(double2), st_b = (size_t)B * sizeof(TreeState);
-    char* sbuf = nullptr;
-    SH_HIP(hipMallocAsync((void**)&sbuf, part_b + st_b + (size_t)B * kDrawChunks * sizeof(double), e->stream));
+    void* sv = nullptr;
+    if (int rc = sh_engine_scratch(e, SCR_TREE, part_b + st_b + (size_t)B * kDrawChunks * sizeof(double), &sv)) return rc;
+    char* sbuf = (char*)sv;
     double2* part = reinterpret_cast<double2*>(sbuf);
     TreeState* st = reinterpret_cast<TreeState*>(sbuf + part_b);
     double* chunk = reinterpret_cast<double*>(sbuf + part_b + st_b);
@@ -1509,11 +1510,8 @@ extern "C" int sh_tree_accept(sh_engine* e, const float* p_logits_dev, const flo
                            B, n, V, inv_t, part, nch, st, chunk);
     }
     le = hipGetLastError();
-    (void)hipFreeAsync(sbuf, e->stream);
   }
   sh_prof_end(e, "tree_accept", 4.0 * V * B * n * (greedy ? 1 : 2), ev);
-  if (udev) (void)hipFreeAsync(udev, e->stream);
-  if (r) (void)hipFreeAsync(r, e->stream);
   SH_CHECK(le == hipSuccess, SH_ERR_HIP, "tree_accept launch: %s", hipGetErrorString(le));
   SH_HIP(hipStreamSynchronize(e->stream));
   return sh_prof_flush(e);

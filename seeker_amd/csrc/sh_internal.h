@@ -118,15 +118,34 @@ struct sh_engine {
   std::vector<GraphEntry> graphs;
   // Device scratch kept by the engine and reused by later calls (the engine
   // stream orders them): grown on demand by sh_engine_scratch.
-  void* scr[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
-  size_t scr_bytes[5] = {0, 0, 0, 0, 0};
+  void* scr[11] = {};
+  size_t scr_bytes[11] = {};
   uint64_t graph_captures = 0, graph_launches = 0;  // replay counters (sh_engine_graph_stats)
 };
 // Scratch slots of sh_engine_scratch.
-enum ScratchSlot { SCR_ACCEPT = 0, SCR_UNIFORMS = 1, SCR_TREE = 2, SCR_SMALL = 3, SCR_WIDE = 4, SCR_SLOTS = 5 };
+// A call's block stays valid until the next call
+// that takes the same slot on this engine (the stream orders them): WIDE a wide
+// forward's activations, COLS a forward call's tokens, masks and ids, FAB a
+// chunk's batched-attention tables, ROWS the samplers' rows, VERIFY the logits
+// and tables of a verify that keeps them, GEMV / XS the kernel-level products
+// (XS apart: its unused lanes are zeroed when it grows and never written).
+// Captured graphs point into none of those from WIDE on.
+enum ScratchSlot {
+  SCR_ACCEPT = 0, SCR_UNIFORMS = 1, SCR_TREE = 2, SCR_SMALL = 3, SCR_WIDE = 4, SCR_COLS = 5, SCR_FAB = 6, SCR_ROWS = 7,
+  SCR_VERIFY = 8, SCR_GEMV = 9, SCR_XS = 10, SCR_SLOTS = 11
+};
 // *out = the engine's scratch of slot, at least `bytes` long. Growing it
 // waits for the stream (earlier launches may still read the old block).
 int sh_engine_scratch(sh_engine* e, int slot, size_t bytes, void** out);
+// Byte offsets of the pieces of one scratch block, 256-byte aligned.
+struct ScratchLayout {
+  size_t bytes = 0;
+  size_t take(size_t n) {
+    const size_t o = bytes;
+    bytes += (n + 255) / 256 * 256;
+    return o;
+  }
+};
 
 // A weight matrix on the device, repacked into MFMA tiles.
 struct QMat {
@@ -564,7 +583,7 @@ struct FabSeg {  // device descriptor of a segment
   uint32_t max_seq, kvlen, mask_base, col0, ncol, rows_pad, nsplit;
 };
 struct FabLaunch {
-  uint8_t* dev = nullptr;  // device tables (segments, work items, column -> segment, masks)
+  uint8_t* dev = nullptr;  // device tables in the engine's scratch (segments, work items, column -> segment, masks)
   const FabSeg* segs = nullptr;
   const uint32_t* work = nullptr;    // (segment << 16 | key split) per workgroup
   const uint32_t* colseg = nullptr;  // segment of each chunk column
@@ -575,7 +594,6 @@ struct FabLaunch {
 int sh_fab_plan(sh_engine* e, sh_model* m, const FabSegIn* in, uint32_t nseg, uint32_t nc, FabLaunch* out);
 int sh_fab_launch(sh_engine* e, const sh_model* m, const FabLaunch& fl, uint32_t layer, const float* q, float* attn_out,
                   uint16_t* bx, uint16_t* xs, float* cs, uint16_t* bh = nullptr);
-void sh_fab_free(sh_engine* e, FabLaunch& fl);
 int sh_argmax_launch(sh_engine* e, const float* logits, uint32_t V, uint32_t N, unsigned long long* keys,
                      uint32_t* out_ids);
 // Draws one token per row from softmax(logits / T) by the vocab-order inverse
@@ -634,7 +652,8 @@ int sh_accept_launch(sh_engine* e, const float* p_logits, const float* q_logits,
                      uint32_t k, uint32_t V, const sh_sampling* s, uint64_t counter, const float* uniforms_dev,
                      uint32_t* acc_len, uint32_t* next_tok, void* scratch = nullptr, double* probs_out = nullptr,
                      const uint64_t* rng_dev = nullptr);
-int sh_kv_compact_launch(sh_engine* e, sh_kv* kv, uint32_t base, const uint32_t* src_dev, uint32_t n);
+// stage: n rows of every layer and kv head, K and V.
+int sh_kv_compact_launch(sh_engine* e, sh_kv* kv, uint32_t base, const uint32_t* src_dev, uint32_t n, uint16_t* stage);
 
 // Profiling helpers (no-ops unless e->profiling).
 void sh_prof_begin(sh_engine* e, hipEvent_t* a);
