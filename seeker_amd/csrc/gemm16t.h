@@ -471,11 +471,14 @@ __global__ __launch_bounds__(64 * kWaves, 1) void k_gemm16t(const uint8_t* __res
     // V rows go out with the lanes along the columns: consecutive keys of a row
     // are neighbours in the cache's transposed blocks
     if (tile0 >= tiles) return;
+    QkvColDev tv[CG];
+#pragma unroll
+    for (int c = 0; c < CG; ++c) tv[c] = ea.tab[min(col0 + 32 * c + (lane & 31), N - 1)];
 #pragma unroll
     for (int c = 0; c < CG; ++c) {
       const uint32_t col = col0 + 32 * c + (lane & 31);
       if (col >= N) continue;
-      const QkvColDev t = ea.tab[col];
+      const QkvColDev t = tv[c];
 #pragma unroll
       for (int p = 0; p < TP; ++p)
 #pragma unroll
@@ -483,8 +486,8 @@ __global__ __launch_bounds__(64 * kWaves, 1) void k_gemm16t(const uint8_t* __res
           if (tile0 + 2 * p + q / 2 >= tiles) continue;
           const f16v& a4 = acc[p][c];
           const float v[4] = {a4[4 * q], a4[4 * q + 1], a4[4 * q + 2], a4[4 * q + 3]};
-          qkv_store4(ea, ea.row_base + (tile0 + 2 * p) * 16 + 8 * q + 4 * kh, v, t.pos, t.slot, t.mseq, t.kc, t.vc,
-                     nullptr);
+          qkv_store4(ea, ea.row_base + (tile0 + 2 * p) * 16 + 8 * q + 4 * kh, v, float2{}, float2{}, t.slot, t.mseq,
+                     t.kc, t.vc, nullptr);
         }
     }
     return;
@@ -524,17 +527,39 @@ __global__ __launch_bounds__(64 * kWaves, 1) void k_gemm16t(const uint8_t* __res
       __builtin_amdgcn_wave_barrier();
       continue;
     }
+    if (EPI == EPI_QKV) {
+      // q and k rows: the 8 columns' table entries, then their rotations, all in
+      // flight before the first is used (one by one a group waited for 16 loads
+      // in turn: 6144 x 4096 x 2048 columns 150 -> 136 us, a 2048-column pass of two
+      // 8B layers 2357 -> 2315 us)
+      const uint32_t i0 = (ea.row_base + row0) % ea.hd;
+      QkvColDev t[8];
+      float2 cs[8][2];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) t[i] = ea.tab[min(col0 + 32 * c + 4 * i + (lane >> 4), N - 1)];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float2* rp = ea.rope + (size_t)t[i].pos * (ea.hd / 2) + i0 / 2;
+        cs[i][0] = rp[0];
+        cs[i][1] = rp[1];
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t lc = 4 * i + (lane >> 4), col = col0 + 32 * c + lc;
+        const float4 v = *(const float4*)(st + lc * kLd + er);
+        if (col >= N || row0 >= tiles * 16) continue;
+        const float o[4] = {v.x, v.y, v.z, v.w};
+        qkv_store4(ea, ea.row_base + row0, o, cs[i][0], cs[i][1], t[i].slot, t[i].mseq, t[i].kc, t[i].vc,
+                   ea.out + (size_t)col * ea.Dq);
+      }
+      __builtin_amdgcn_wave_barrier();
+      continue;
+    }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const uint32_t lc = 4 * i + (lane >> 4), col = col0 + 32 * c + lc;
       const float4 v = *(const float4*)(st + lc * kLd + er);
       if (col >= N || row0 >= tiles * 16) continue;
-      if (EPI == EPI_QKV) {
-        const QkvColDev t = ea.tab[col];
-        const float o[4] = {v.x, v.y, v.z, v.w};
-        qkv_store4(ea, ea.row_base + row0, o, t.pos, t.slot, t.mseq, t.kc, t.vc, ea.out + (size_t)col * ea.Dq);
-        continue;
-      }
       float* out = ea.out + (size_t)col * ea.ldo + row0;
       if (EPI == EPI_PART) {
         *(float4*)(out + ks * ea.part_stride) = v;
