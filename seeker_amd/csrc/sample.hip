@@ -580,12 +580,24 @@ __device__ uint32_t sample_filtered_row(const float* __restrict__ x, uint32_t V,
 // chunk whose running sum reaches u * total and draws inside it, as
 // k_sample_cols does over the whole row (first v whose running sum reaches
 // u * total).
+//
+// With seq.drafts (sequences of k + 1 <= 64 rows) the sequence's last row to be
+// drawn also decides it: accepted while sample == draft, the next token the sample
+// after them, as k_decide_compare.
 constexpr uint32_t kSampChunks = 64;
+struct CompareSeq {
+  const uint32_t* drafts;  // [B][k], null: no decision
+  uint32_t k;
+  uint32_t* cnt;  // [B] arrival counters, kCntStride apart, zeroed by k_row_part
+  uint32_t* acc_len;
+  uint32_t* next_tok;
+};
 __global__ __launch_bounds__(256) void k_sample_chunks(const float* __restrict__ p, const double2* __restrict__ part,
                                                        uint32_t nch, uint32_t V, double inv_t, const float* u_dev,
                                                        uint64_t seed, uint64_t word0, uint64_t wstride,
                                                        double2* __restrict__ csum, uint32_t* __restrict__ cnt,
-                                                       uint32_t* __restrict__ out, const uint64_t* rng) {
+                                                       uint32_t* __restrict__ out, const uint64_t* rng,
+                                                       const CompareSeq seq) {
   static_assert(kSampChunks == 64, "one lane per chunk");
   constexpr int kPer = 8;  // elements per thread per pass
   __shared__ double tab[64];
@@ -655,7 +667,33 @@ __global__ __launch_bounds__(256) void k_sample_chunks(const float* __restrict__
   __syncthreads();
   const uint32_t plo = min(s_c * CH, V), phi = min(plo + CH, V);
   const uint32_t tok = wg_inverse_cdf(rw, plo, phi, false, 0.f, s_off, s_target, true, nullptr);
-  if (t == 0) out[row] = tok;
+  if (!seq.drafts) {
+    if (t == 0) out[row] = tok;
+    return;
+  }
+  if (t >= 64) return;
+  const uint32_t b = row / (seq.k + 1);
+  uint32_t last = 0;
+  if (t == 0) {
+    sh_st_coh4(out + row, tok);
+    sh_stores_done();
+    uint32_t* cr = seq.cnt + (size_t)b * kCntStride;
+    last = __hip_atomic_fetch_add(cr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == seq.k;
+    if (last) __hip_atomic_store(cr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (!__shfl(last, 0)) return;
+  // lane i < k: sample i against draft i; lane k (k <= 63) holds the last sample
+  const uint32_t* so = out + (size_t)b * (seq.k + 1);
+  uint32_t si = sh_ld_coh4(so + min(t, seq.k));
+  sh_coh_wait(si);
+  const bool miss = t < seq.k && si != seq.drafts[(size_t)b * seq.k + t];
+  const unsigned long long m = __ballot(miss);
+  const uint32_t i = m ? (uint32_t)__builtin_ctzll(m) : seq.k;
+  const uint32_t nx = __shfl(si, i);
+  if (t == 0) {
+    seq.acc_len[b] = i;
+    seq.next_tok[b] = nx;
+  }
 }
 
 // COMPARE with filters: row r of p draws with Philox word word0 + wstride r
@@ -1197,6 +1235,13 @@ __global__ __launch_bounds__(256) void k_tree_pass(const float* __restrict__ p, 
 
 // Rows of at least this many logits draw through k_sample_chunks.
 constexpr uint32_t kChunkedMinV = 8192;
+// COMPARE calls of at most this many rows are decided inside the draw: a launch
+// less, where the call is launches and latency (5 rows of 32000 13.2 -> 12.8 us,
+// 9 of 151936 18.3 -> 18.1, 40 of 32000 19.2 -> 19.0). With many rows the second
+// arrival costs more than the launch (288 rows of 128256 120.8 -> 121.7, 640 of
+// 32000 157.5 -> 162.4). The same for REJECTION, the pick inside k_draw_chunks,
+// took 33 us instead of 26 for 32 sequences of 128256, and is not done.
+constexpr uint32_t kDecideInDrawRows = 64;
 static size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 // The chunked draw's chunk sums and arrival counters for nrows rows.
 static size_t chunked_bytes(uint32_t nrows) {
@@ -1209,7 +1254,9 @@ size_t sh_accept_scratch_bytes(uint32_t B, uint32_t k, uint32_t V, uint32_t mode
   const size_t part_b = (size_t)(n_p + n_q) * nch * sizeof(double2);
   const size_t chunk_b = (size_t)B * kDrawChunks * sizeof(double2), rstat_b = (size_t)B * 2 * sizeof(double2);
   const size_t small_b = mode == SH_SAMPLE_COMPARE ? (size_t)n_p * 4 : (size_t)B * 4;
-  const size_t samp_b = mode == SH_SAMPLE_COMPARE && V >= kChunkedMinV ? chunked_bytes(n_p) : 0;
+  // the chunked COMPARE draw, and the arrival counters of the B sequences
+  const size_t samp_b =
+      mode == SH_SAMPLE_COMPARE && V >= kChunkedMinV ? chunked_bytes(n_p) + (size_t)B * kCntStride * 4 : 0;
   return round256(part_b + chunk_b + rstat_b + round256(small_b)) + samp_b;
 }
 
@@ -1222,12 +1269,13 @@ size_t sh_sample_rows_scratch_bytes(uint32_t nrows, uint32_t V) {
 // wide rows in kSampChunks chunks per row (scratch at samp: chunked_bytes).
 static void launch_sample_cols(sh_engine* e, const float* p, const double2* part, uint32_t nch, uint32_t nrows,
                                uint32_t V, double inv_t, const float* u_dev, uint64_t seed, uint64_t word0,
-                               uint64_t wstride, char* samp, uint32_t* out, const uint64_t* rng) {
+                               uint64_t wstride, char* samp, uint32_t* out, const uint64_t* rng,
+                               const CompareSeq& seq = CompareSeq{}) {
   if (V >= kChunkedMinV) {
     double2* csum = reinterpret_cast<double2*>(samp);
     uint32_t* cnt = reinterpret_cast<uint32_t*>(samp + round256((size_t)nrows * kSampChunks * sizeof(double2)));
     hipLaunchKernelGGL(k_sample_chunks, dim3(kSampChunks, nrows), dim3(256), 0, e->stream, p, part, nch, V, inv_t,
-                       u_dev, seed, word0, wstride, csum, cnt, out, rng);
+                       u_dev, seed, word0, wstride, csum, cnt, out, rng, seq);
   } else {
     hipLaunchKernelGGL(k_sample_cols, dim3(nrows), dim3(256), 0, e->stream, p, part, nch, V, inv_t, u_dev, seed,
                        word0, wstride, out, rng);
@@ -1271,15 +1319,20 @@ int sh_accept_launch(sh_engine* e, const float* p_logits, const float* q_logits,
   const size_t small_b = mode == SH_SAMPLE_COMPARE ? (size_t)n_p * 4 : (size_t)B * 4;
   char* samp = sbuf + round256(part_b + chunk_b + rstat_b + round256(small_b));  // the chunked COMPARE draw
   uint32_t* zc = mode == SH_SAMPLE_COMPARE ? sample_cols_cnt(samp, n_p, V) : nullptr;
+  // the sequences' counters follow the rows' when the draw decides
+  const bool in_draw = zc && n_p <= kDecideInDrawRows;
+  const uint32_t nzero = in_draw ? n_p + B : n_p;
+  const CompareSeq seq = in_draw ? CompareSeq{drafts, k, zc + (size_t)n_p * kCntStride, acc_len, next_tok}
+                                 : CompareSeq{};
   hipEvent_t ev = nullptr;
   sh_prof_begin(e, &ev);
   if (filt.top_k) {  // the filtered draw reads its rows itself
   } else if (V % 4 == 0) {
     hipLaunchKernelGGL((k_row_part<true, kStatE>), dim3(nunits), dim3(256), 0, e->stream, p_logits, n_p, q_logits,
-                       V, inv_t, nch, part, nullptr, zc, n_p);
+                       V, inv_t, nch, part, nullptr, zc, nzero);
   } else {
     hipLaunchKernelGGL((k_row_part<false, kStatE>), dim3(nunits), dim3(256), 0, e->stream, p_logits, n_p, q_logits,
-                       V, inv_t, nch, part, nullptr, zc, n_p);
+                       V, inv_t, nch, part, nullptr, zc, nzero);
   }
   SH_HIP(hipGetLastError());
   sh_prof_end(e, "accept_stats", 4.0 * V * (n_p + n_q), ev);
@@ -1292,9 +1345,10 @@ int sh_accept_launch(sh_engine* e, const float* p_logits, const float* q_logits,
                        next_tok);
   } else if (mode == SH_SAMPLE_COMPARE) {
     launch_sample_cols(e, p_logits, part, nch, n_p, V, inv_t, uniforms_dev, s->seed, counter + 1ull, 2ull, samp,
-                       small, rng_dev);
-    hipLaunchKernelGGL(k_decide_compare, dim3((B + 63) / 64), dim3(64), 0, e->stream, small, drafts, B, k, acc_len,
-                       next_tok);
+                       small, rng_dev, seq);
+    if (!in_draw)
+      hipLaunchKernelGGL(k_decide_compare, dim3((B + 63) / 64), dim3(64), 0, e->stream, small, drafts, B, k, acc_len,
+                         next_tok);
   } else {
     hipLaunchKernelGGL(k_decide_reject, dim3(B), dim3(256), 0, e->stream, p_logits, q_logits, part, nch, B, k, V,
                        inv_t, drafts, uniforms_dev, s->seed, counter, small, rstat, probs_out, rng_dev);
