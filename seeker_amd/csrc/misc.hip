@@ -287,18 +287,23 @@ int sh_part_reduce_launch(sh_engine* e, const float* part, uint32_t nparts, uint
 
 // ------------------------------------------------------------------ argmax
 
-// One kernel per argmax: each workgroup folds its 2048-logit block into the
-// column's key (atomic max), then counts itself in on its column's counter;
+// One kernel per argmax: each workgroup folds its block of 256 PER_T logits into
+// the column's key (atomic max), then counts itself in on its column's counter;
 // the column's last workgroup to arrive writes its id and clears the key and
 // the counter for the next launch (zero at allocation, so graph replays need
-// no memset). The counters follow the SH_MAX_COLS keys, 64 bytes apart (one
-// shared counter serialised every workgroup's arrival: 9.9 us for 8 columns).
+// no memset). Bound by those atomics, which the memory side takes one after the
+// other within a cache line (~20 ns each): keys and counters lie 64 bytes apart
+// in two regions of SH_MAX_COLS16 columns, and calls of many blocks take larger
+// ones (164 columns of 32000: three launches of 64 columns and 2048-logit blocks
+// with 8 keys a line 20.7 us, one launch 9.9 us; 56 columns 7.6 -> 6.1 us).
+template <uint32_t PER_T>
 __global__ __launch_bounds__(256) void k_argmax(const float* __restrict__ logits, uint32_t V, uint32_t N,
                                                 unsigned long long* keys, uint32_t* __restrict__ out) {
   const uint32_t col = blockIdx.y;
   const float* row = logits + (size_t)col * V;
+  unsigned long long* key = keys + 8 * col;
   unsigned long long best = 0ull;
-  constexpr uint32_t PER_T = 8, per = 256 * PER_T;
+  constexpr uint32_t per = 256 * PER_T;
   const uint32_t i0 = blockIdx.x * per;
   const uint32_t i1 = min(i0 + per, V);
   // every load of the thread goes out before the first compare (one round trip)
@@ -324,16 +329,16 @@ __global__ __launch_bounds__(256) void k_argmax(const float* __restrict__ logits
     for (int w = 1; w < 4; ++w) best = wb[w] > best ? wb[w] : best;
     // the returned value orders the max before the arrival
     const unsigned long long prev =
-        __hip_atomic_fetch_max(keys + col, best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_fetch_max(key, best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     asm volatile("s_waitcnt vmcnt(0)" : : "v"(prev) : "memory");
-    uint32_t* cnt = (uint32_t*)(keys + SH_MAX_COLS + 8 * col);
+    uint32_t* cnt = (uint32_t*)(key + 8 * SH_MAX_COLS16);
     const uint32_t arrived = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
     const bool last = arrived == gridDim.x;
     if (last) {
       __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const unsigned long long k = __hip_atomic_load(keys + col, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const unsigned long long k = __hip_atomic_load(key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       out[col] = sh_amax_index(k);
-      __hip_atomic_store(keys + col, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(key, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
 }
@@ -343,11 +348,11 @@ int sh_argmax_launch(sh_engine* e, const float* logits, uint32_t V, uint32_t N, 
   SH_CHECK(N >= 1 && N <= SH_MAX_COLS16, SH_ERR_ARG, "argmax N=%u", N);
   hipEvent_t ev = nullptr;
   sh_prof_begin(e, &ev);
-  for (uint32_t c0 = 0; c0 < N; c0 += SH_MAX_COLS) {  // SH_MAX_COLS keys: launches of at most that many columns
-    const uint32_t n = std::min<uint32_t>(SH_MAX_COLS, N - c0);
-    hipLaunchKernelGGL(k_argmax, dim3((V + 2047) / 2048, n), dim3(256), 0, e->stream, logits + (size_t)c0 * V, V, n,
-                       keys, out_ids + c0);
-  }
+  // 8192-logit blocks where they still give every CU two workgroups
+  if ((uint64_t)N * ((V + 8191) / 8192) >= 512)
+    hipLaunchKernelGGL(k_argmax<32>, dim3((V + 8191) / 8192, N), dim3(256), 0, e->stream, logits, V, N, keys, out_ids);
+  else
+    hipLaunchKernelGGL(k_argmax<8>, dim3((V + 2047) / 2048, N), dim3(256), 0, e->stream, logits, V, N, keys, out_ids);
   SH_HIP(hipGetLastError());
   sh_prof_end(e, "argmax", 4.0 * V * N, ev);
   return SH_OK;

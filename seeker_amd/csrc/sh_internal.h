@@ -57,14 +57,14 @@ __host__ __device__ constexpr bool sh_is_kquant(int type) {
   return type == GGML_Q4_K || type == GGML_Q5_K || type == GGML_Q6_K;
 }
 constexpr uint32_t SH_MAX_COLS = 64;     // columns per forward chunk (8 operand groups of 8)
-// argmax workspace (64-bit words): SH_MAX_COLS keys, then one arrival counter
-// per column, 64 bytes apart
-constexpr uint32_t SH_AMAX_WORDS = SH_MAX_COLS + 8 * SH_MAX_COLS;
 constexpr uint32_t SH_MAX_PREP_COLS = 512;  // operand columns one prep builds (the MoE down operand: pairs)
 constexpr int SH_FA_MIN_SPLIT_KEYS = 64;  // smallest key split of any attention launch (sizes fa_part)
 constexpr uint32_t SH_WIDE16_COLS = 32;  // the reference's wide-GEMM threshold (ops/matmul.rs:433-446)
 constexpr uint32_t SH_MAX_COLS16 = 192;  // columns per forward chunk of a wide f16 call (12 MFMA groups of 16)
 constexpr uint32_t SH_MAX_COLS_T = 2048;  // columns of one pass of the large-tile wide GEMM (k_gemm16t)
+// argmax workspace (64-bit words): SH_MAX_COLS16 keys, then as many arrival
+// counters, each 64 bytes apart
+constexpr uint32_t SH_AMAX_WORDS = 2 * 8 * SH_MAX_COLS16;
 constexpr size_t SH_PART16_BYTES = 64u << 20;  // most split partials of a wide f16 GEMM (above, fewer splits)
 constexpr int SH_FA_MAX_ROWS = 256;       // padded query rows (gqa x columns) per kv head
 // Split partial row: O[hd], m, l, 2 pad (keeps rows 16-byte aligned).
